@@ -1,0 +1,374 @@
+"""The workloads by which this framework's speed is measured.
+
+Each case is one call (or one step) of what a program does with the package
+through its public entry points: the Poisson solves of the aligned hierarchy,
+implicit convection-diffusion-reaction steps in the reference's arithmetic,
+Scharfetter-Gummel species steps and their adjoint, whole steps of the
+discharge and plasma drivers, and the transport assembly between the solves.
+``listed()`` names the cases, ``draw(rng)`` gives others of the same ranges,
+``prepare`` makes the inputs and the contexts that a program keeps, ``run``
+does one pass, ``work`` says what a pass cannot do without, and ``exact``
+gives the results in 64 bits where plain torch can.
+"""
+import math
+
+import torch
+
+from mps3d_amd import FieldSolver
+from mps3d_amd import chemistry, discharge, plasma
+from mps3d_amd import workloads as W
+from mps3d_amd.autograd import Operator, linear_solve
+
+DEV = "cuda"
+F64 = torch.float64
+PLATES = ("ZGRD", "ZGRD", "ZGRD", "ZGRD", "DIRC", "DIRC")
+DECKS = {"ion_elec": (plasma.ION_ELEC_DECK, chemistry.ion_elec), "h2_o2": (plasma.H2_O2_DECK, chemistry.h2_o2)}
+
+
+def listed():
+    return [
+        # a small re-solve of the potential, once per time step of a small model
+        {"name": "poisson_33_fp64", "kind": "poisson", "nx": 33, "ny": 33, "nz": 33, "precision": "fp64"},
+        # an ordinary gap with unequal sides, in plain FP64
+        {"name": "poisson_161x97x129_fp64", "kind": "poisson", "nx": 161, "ny": 97, "nz": 129,
+         "precision": "fp64"},
+        # the benchmark: FP32 smoothing under FP64 defect correction at 257^3
+        {"name": "poisson_257_fp32dc", "kind": "poisson", "nx": 257, "ny": 257, "nz": 257,
+         "precision": "fp32dc"},
+        # one implicit step of the generic-PDE deck at its own size, in the reference's arithmetic
+        {"name": "cdr_80x48x32", "kind": "cdr", "nx": 80, "ny": 48, "nz": 32, "px": 5, "py": 3, "pz": 2},
+        # the same step on a large grid
+        {"name": "cdr_128", "kind": "cdr", "nx": 128, "ny": 128, "nz": 128, "px": 2, "py": 2, "pz": 4},
+        # a species step of an optimisation: forward solve and the gradients of its inputs
+        {"name": "drift_grad_65_fp64", "kind": "drift", "nx": 65, "ny": 65, "nz": 65, "precision": "fp64",
+         "hierarchy": "aligned", "grad": True},
+        # a species step of a large model, forward only
+        {"name": "drift_193x129x161_fp32dc", "kind": "drift", "nx": 193, "ny": 129, "nz": 161,
+         "precision": "fp32dc", "hierarchy": "aligned", "grad": False},
+        # one step of the coupled glow discharge (Poisson, two species, electron energy)
+        {"name": "glow_step_128", "kind": "glow", "n": 128, "p": 1, "volts": 1000.0},
+        # one step of the five-species discharge
+        {"name": "five_species_step_129", "kind": "five", "n": 129, "volts": 800.0},
+        # one time step of the plasma decks: their own size, and a larger domain
+        {"name": "plasma_h2_o2_32", "kind": "plasma", "chem": "h2_o2", "nx": 32, "ny": 32, "nz": 32,
+         "px": 2, "py": 4, "pz": 1, "volts": 1.0},
+        {"name": "plasma_ion_elec_96x128x64", "kind": "plasma", "chem": "ion_elec", "nx": 96, "ny": 128, "nz": 64,
+         "px": 3, "py": 4, "pz": 2, "volts": 1.0},
+        # the field and the coefficient assembly of one step, on a grid of no special size
+        {"name": "transport_187x150x131", "kind": "transport", "chem": "ion_elec", "nx": 187, "ny": 150, "nz": 131},
+    ]
+
+
+def draw(rng):
+    kind = rng.choice(["poisson", "poisson", "cdr", "drift", "drift", "glow", "five", "plasma", "plasma", "transport"])
+    if kind in ("poisson", "drift"):
+        # sizes m 2^k + 1, up to 257 (Poisson) and 193 (drift) a side
+        k = rng.choice([4, 5, 5])
+        top = 7 if kind == "poisson" else 6
+        nx, ny, nz = (rng.randint(1 if k == 5 else 2, top) * 2 ** k + 1 for _ in range(3))
+        c = {"kind": kind, "nx": nx, "ny": ny, "nz": nz, "precision": rng.choice(["fp32dc", "fp64"])}
+        if kind == "drift":
+            c.update(hierarchy="aligned", grad=rng.random() < 0.4 and nx * ny * nz < 10 ** 6)
+        return c
+    if kind == "cdr":
+        p = [rng.randint(1, 4) for _ in range(3)]
+        k = rng.choice([3, 4, 5]) if max(p) < 4 else rng.choice([3, 4])
+        return dict({"kind": kind}, **{"n" + a: q * 2 ** k for a, q in zip("xyz", p)},
+                    **{"p" + a: q for a, q in zip("xyz", p)})
+    volts = round(rng.uniform(400.0, 1200.0), 1)
+    if kind == "glow":
+        p, k = rng.choice([(1, 5), (1, 6), (3, 4), (3, 5), (5, 4), (1, 7)])
+        return {"kind": kind, "n": p * 2 ** k, "p": p, "volts": volts}
+    if kind == "five":
+        return {"kind": kind, "n": rng.choice([33, 49, 65, 81, 97, 113, 129]), "volts": volts}
+    if kind == "plasma":
+        p = rng.choice([(2, 4, 1), (2, 2, 2), (3, 4, 2), (4, 4, 2), (3, 2, 5), (2, 3, 1)])
+        k = rng.choice([3, 4]) if max(p) > 3 else rng.choice([3, 4, 5])
+        return dict({"kind": kind, "chem": rng.choice(["ion_elec", "h2_o2"]), "volts": round(volts / 1000, 3)},
+                    **{"n" + a: q * 2 ** k * (2 if q == 1 else 1) for a, q in zip("xyz", p)},
+                    **{"p" + a: q for a, q in zip("xyz", p)})
+    nx, ny, nz = (int(round(math.exp(rng.uniform(math.log(17), math.log(136))))) for _ in range(3))
+    return {"kind": kind, "chem": rng.choice(["ion_elec", "h2_o2"]), "nx": nx, "ny": ny, "nz": nz}
+
+
+# ------------------------------------------------------------------ inputs
+def _size(c):
+    return (c["n"],) * 3 if "n" in c else (c["nx"], c["ny"], c["nz"])
+
+
+def _gen(seed):
+    return torch.Generator(device="cpu").manual_seed(int(seed))
+
+
+def _pad(t):
+    return torch.nn.functional.pad(t, (1,) * 6).contiguous()
+
+
+def _centres(n, length):
+    """Cell-centre coordinates, broadcastable over (nz, ny, nx)."""
+    x, y, z = ((torch.arange(m, dtype=F64, device=DEV) + 0.5) * (L / m) for m, L in zip(n, length))
+    return x[None, None, :], y[None, :, None], z[:, None, None]
+
+
+def _waves(n, gen, modes=4):
+    """A smooth random (nz, ny, nx) field: products of low cosine modes that
+    have zero normal gradient on the domain's faces."""
+    x, y, z = _centres(n, (1.0, 1.0, 1.0))
+    f = torch.zeros(n[::-1], dtype=F64, device=DEV)
+    for _ in range(modes):
+        a, k = torch.randn(1, generator=gen).item(), torch.randint(0, 4, (3,), generator=gen).tolist()
+        f += a * torch.cos(math.pi * k[0] * x) * torch.cos(math.pi * k[1] * y) * torch.cos(math.pi * k[2] * z)
+    return f
+
+
+def _poisson_inputs(c, seed):
+    """Length per side, permittivity (a slab of 4 on a quarter of the gap),
+    space charge of seeded blobs over eps0 and the upper plate's potential."""
+    n = _size(c)
+    length = tuple(0.02 * m / max(n) for m in n)
+    x, y, z = _centres(n, length)
+    eps = torch.where(z < 0.25 * length[2], 4.0, 1.0).to(F64).expand(n[::-1]).contiguous()
+    rho = torch.zeros(n[::-1], dtype=F64, device=DEV)
+    for cx, cy, cz, s, a in W.blob_params(seed, length=1.0):
+        rho += a * torch.exp(-((x - cx * length[0]) ** 2 + (y - cy * length[1]) ** 2 + (z - cz * length[2]) ** 2)
+                             / (2 * s * s))
+    return length, eps, rho * (W.E_CHARGE / W.EPS0), 1000.0
+
+
+def _cdr_inputs(c, seed):
+    """The generic-PDE deck (velocity -1 along x, D = 0.5, reaction 2, dt 0.1;
+    cubic cells) and the field of the time step before."""
+    n = _size(c)
+    length = tuple(m / n[0] for m in n)
+    x, _, _ = _centres(n, length)
+    old = (x * x - x) / 2 + 0.05 * _waves(n, _gen(seed))
+    return length, -(x * x).expand(n[::-1]).contiguous(), old.contiguous()
+
+
+def _drift_inputs(c, seed):
+    """Electron drift in a 2 cm gap at 1 kV plus a smooth space-charge field."""
+    n, g = _size(c), _gen(seed)
+    length = tuple(0.02 * m / max(n) for m in n)
+    pot = 40.0 * _waves(n, g)
+    q = torch.nn.functional.pad(pot[None], (1,) * 6, mode="replicate")[0]
+    h = [L / m for L, m in zip(length, n)]
+    ex = (q[1:-1, 1:-1, :-2] - q[1:-1, 1:-1, 2:]) / (2 * h[0])
+    ey = (q[1:-1, :-2, 1:-1] - q[1:-1, 2:, 1:-1]) / (2 * h[1])
+    ez = (q[:-2, 1:-1, 1:-1] - q[2:, 1:-1, 1:-1]) / (2 * h[2]) - 1000.0 / length[2]
+    vel = [(-20.0 * e).contiguous() for e in (ex, ey, ez)]
+    x, y, z = _centres(n, length)
+    r2 = sum((t - L / 2) ** 2 for t, L in zip((x, y, z), length))
+    dens = (1e13 + 1e16 * torch.exp(-r2 / (2 * 1e-3 ** 2))) * (1.0 + 0.1 * torch.tanh(_waves(n, g)))
+    rhs = dens / 1e-11 + 1e23 * torch.exp(-r2 / (2 * 2e-3 ** 2))
+    return length, dens, rhs, vel, torch.tanh(_waves(n, g))
+
+
+def _deck(c, seed):
+    """The deck with the case's grid and part of its voltage and, by the seed,
+    its plasma density and electron temperature."""
+    deck, chem = DECKS[c["chem"]]
+    f = 0.5 + torch.rand(2, generator=_gen(seed)).double()
+    d = dict(deck, n=_size(c), p=(c["px"], c["py"], c["pz"]))
+    skip = ("N", "H2", "O2", "POT", "ELECTEMP")
+    d["init"] = {k: v if k in skip else v * f[0].item() for k, v in deck["init"].items()}
+    d["init"]["ELECTEMP"] *= f[1].item()
+    d["bcs"] = [b[:7] + (b[7] * c["volts"],) + b[8:] for b in deck["bcs"]]
+    return d, chem()
+
+
+def prepare(case, seed):
+    kind, n = case["kind"], _size(case)
+    if kind == "poisson":
+        length, eps, source, volts = _poisson_inputs(case, seed)
+        s = FieldSolver(n, length, hierarchy="aligned", precision=case["precision"], max_cycles=40, tol=1e-10,
+                        tol_kind="rel", arith="fast", start="fmg")
+        s.set_bc(PLATES, (0.0, 0.0, 0.0, 0.0, 0.0, volts))
+        s.set_coeffs(_pad(eps), source=_pad(source))
+        return {"case": case, "solver": s, "source": _pad(source), "u": torch.zeros(s.shape[::-1], dtype=F64, device=DEV)}
+    if kind == "cdr":
+        length, base, old = _cdr_inputs(case, seed)
+        s = FieldSolver(n, length, p=(case["px"], case["py"], case["pz"]))
+        s.set_bc(("DIRC", "FLUX", "ZGRD", "ZGRD", "ZGRD", "ZGRD"), (0.0, -0.25, 0.0, 0.0, 0.0, 0.0))
+        one = torch.ones(n[::-1], dtype=F64, device=DEV)
+        s.set_coeffs(_pad(0.5 * one), _pad(-one), _pad(0 * one), _pad(0 * one), _pad(2.0 * one), None, True, 0.1)
+        old = _pad(old)
+        return {"case": case, "solver": s, "base": _pad(base), "old": old, "u": old.clone(), "src": torch.empty_like(old)}
+    if kind == "drift":
+        length, dens, rhs, vel, g = _drift_inputs(case, seed)
+        op = Operator(n, length, torch.full(n[::-1], 100.0, dtype=F64, device=DEV),
+                      ("ZGRD",) * 4 + ("FLUX", "FLUX"), flux="sg", timederiv=True, dt=1e-11, tol=1e-10,
+                      method="gmres", hierarchy=case["hierarchy"], precision=case["precision"], arith="fast")
+        for t in [rhs] + vel:
+            t.requires_grad_(case["grad"])
+        return {"case": case, "op": op, "dens": dens, "rhs": rhs, "vel": vel, "g": g}
+    if kind in ("glow", "five"):
+        r = torch.rand(2, generator=_gen(seed)).double()
+        if kind == "glow":
+            p = (case["p"],) * 3
+            model, (dens, neps) = discharge.glow_discharge(n[0], p=p)
+            volts = [case["volts"]]
+        else:
+            model, (dens, neps), _ = discharge.five_species(n[0])
+            volts = [case["volts"], -case["volts"]]
+        f = 0.5 + r[0].item()
+        return {"case": case, "model": model, "dens": tuple(f * d for d in dens),
+                "neps": None if neps is None else f * neps,
+                "V": torch.tensor(volts, dtype=F64, device=DEV) * (0.8 + 0.4 * r[1].item())}
+    if kind == "plasma":
+        deck, chem = _deck(case, seed)
+        return {"case": case, "run": plasma.PlasmaRun(deck, chem)}
+    # transport: physical fields of a developed discharge, on every cell and ghost
+    gen = torch.Generator(device=DEV).manual_seed(int(seed))
+    deck, make = DECKS[case["chem"]]
+    chem, g = make(), tuple(v + 2 for v in n)[::-1]
+
+    def field(lo, hi, m=1):
+        return lo + (hi - lo) * torch.rand((m,) + g, generator=gen, dtype=F64, device=DEV)
+
+    sc = deck["scales"]
+    numden = field(0.5, 2.0, chem.nspecies)
+    for q, nm in enumerate(chem.names):
+        numden[q] *= deck["init"][nm]
+    te = field(5e3, 6e4)[0]
+    eescale = sc["ELECDEN"] * chemistry.K_BMAN * sc["ETEMP"]
+    ne = numden[chem.especnum - 1]
+    s = FieldSolver(n, tuple(L / sc["LENGTH"] for L in deck["length"]))
+    s.set_chemistry(chem)
+    s.set_bc(PLATES, (0.0, 0.0, 0.0, 0.0, 0.0, 1.0))
+    s.set_coeffs(torch.ones(g, dtype=F64, device=DEV))
+    new = lambda m: torch.zeros(m * ne.numel(), dtype=F64, device=DEV)  # noqa: E731
+    outs = [{"vel": new(3), "dcoeff": new(1), "reac": new(1), "source": new(1), "prod": new(1)} for _ in range(3)]
+    return {"case": case, "solver": s, "chem": chem, "sc": sc, "numden": numden, "te": te, "ee": eescale,
+            "eps": 1.5 * chemistry.K_BMAN * ne * te / eescale, "phi": field(0.0, 1.0)[0], "E": new(3), "outs": outs,
+            "ne_s": ne / sc["ELECDEN"]}
+
+
+# -------------------------------------------------------------------- runs
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "poisson":
+        s, u = state["solver"], state["u"]
+        u.zero_()
+        s.set_source(state["source"])
+        s.solve(u, raise_on_failure=True)
+        return u[1:-1, 1:-1, 1:-1]
+    if kind == "cdr":
+        s, u, old = state["solver"], state["u"], state["old"]
+        u.copy_(old)
+        s.set_source(torch.add(state["base"], old, alpha=10.0, out=state["src"]))
+        s.solve(u)
+        s.fill_ghosts(u)
+        return u[1:-1, 1:-1, 1:-1]
+    if kind == "drift":
+        x = linear_solve(state["op"], state["rhs"], tuple(state["vel"]), x0=state["dens"])
+        if not case["grad"]:
+            return {"x": x}
+        grads = torch.autograd.grad(x, [state["rhs"]] + state["vel"], state["g"])
+        return {"x": x.detach(), "grads": list(grads)}
+    if kind in ("glow", "five"):
+        with torch.no_grad():
+            dens, neps = state["model"].step(state["dens"], state["neps"], state["V"])
+        return {"dens": list(dens), "neps": neps, "phi": state["model"]._phi}
+    if kind == "plasma":
+        r = state["run"]
+        r.step()
+        cut = (Ellipsis,) + (slice(1, -1),) * 3
+        return {"numden": r.numden[cut], "pot": r.pot[cut], "E": r.E[cut], "Te": r.Te[cut], "eps": r.eps[cut],
+                "eprod": r.eprod[cut]}
+    s, sc, chem, nd, te = (state[k] for k in ("solver", "sc", "chem", "numden", "te"))
+    e, flat = chem.especnum - 1, nd.view(-1)
+    tl, tl2, t0 = sc["TIME"] / sc["LENGTH"], sc["TIME"] / sc["LENGTH"] ** 2, sc["TIME"]
+    o = state["outs"]
+    ions = nd[chem.ionspecmin - 1:chem.ionspecmax].reshape(-1)
+    s.poisson_transport(nd[e].view(-1), ions, (tl, tl2, t0, t0 / sc["POT"]), timederiv=False, out=o[0])
+    s.efield(state["phi"], sc["POT"] / sc["LENGTH"], out=state["E"])
+    s.eenergy_transport(state["E"], te.view(-1), flat, (tl, tl2, t0, t0 / state["ee"]), lscale=sc["LENGTH"],
+                        soln=state["eps"].view(-1), out=o[1])
+    s.species_transport(chem.especnum, state["E"], te.view(-1), flat, (tl, tl2, t0, t0 / sc["ELECDEN"]),
+                        soln=state["ne_s"].view(-1), out=o[2])
+    s.electron_temp(state["eps"].view(-1), nd[e].view(-1), state["ee"], chemistry.etempmin_default(), te.view(-1))
+    keep = ("vel", "dcoeff", "reac", "source")
+    return {"poisson": {k: o[0][k] for k in keep}, "E": state["E"], "eenergy": {k: o[1][k] for k in keep},
+            "electrons": {k: o[2][k] for k in keep + ("prod",)}, "te": te, "eps": state["eps"]}
+
+
+def work(case):
+    """Bytes: each field that a pass takes and each that it gives, once.
+    Operations: a 7-point row (about 20) per cell and equation."""
+    n = _size(case)
+    cells = n[0] * n[1] * n[2]
+    kind = case["kind"]
+    if kind == "poisson":
+        f, eqs = 3, 1           # source, coefficient, potential
+    elif kind == "cdr":
+        f, eqs = 8, 1           # five coefficients, source, field before and after
+    elif kind == "drift":
+        f, eqs = (13, 2) if case["grad"] else (7, 1)   # D, velocities, right-hand side, guess, result (, gradients)
+    elif kind == "glow":
+        f, eqs = 8, 4
+    elif kind == "five":
+        f, eqs = 12, 6
+    else:
+        _, make = DECKS[case["chem"]]
+        ns = make().nspecies
+        if kind == "plasma":
+            f, eqs = 2 * (ns + 8), (7 if case["chem"] == "h2_o2" else 3) + 3
+        else:
+            f, eqs = 2 * ns + 32, 4
+    return {"bytes": 8.0 * f * cells, "flops": 20.0 * eqs * cells}
+
+
+# ------------------------------------------------------- results in 64 bits
+def _separable(lo, diag, hi, lat, widths, rhs):
+    """Solves a 7-point system with rows (lo, diag, hi) along the first axis
+    and lat[k] times the Neumann Laplacian (cell width widths) along the other
+    two: cosine transforms and one tridiagonal solve per mode."""
+    def cosines(m):
+        j = torch.arange(m, dtype=F64, device=DEV)
+        C = torch.cos(math.pi * j[:, None] * (j[None, :] + 0.5) / m) * math.sqrt(2.0 / m)
+        C[0] /= math.sqrt(2.0)
+        return C, 2.0 - 2.0 * torch.cos(math.pi * j / m)
+
+    n0, n1, n2 = rhs.shape
+    (C1, l1), (C2, l2) = cosines(n1), cosines(n2)
+    f = torch.matmul(torch.matmul(C1, rhs), C2.t().contiguous())
+    lam = l1[:, None] / widths[0] ** 2 + l2[None, :] / widths[1] ** 2
+    up = torch.empty_like(f)
+    for k in range(n0):
+        d = diag[k] + lat[k] * lam
+        if k:
+            d = d - lo[k] * up[k - 1]
+            f[k] -= lo[k] * f[k - 1]
+        up[k] = hi[k] / d
+        f[k] /= d
+    for k in range(n0 - 2, -1, -1):
+        f[k] -= up[k] * f[k + 1]
+    return torch.matmul(torch.matmul(C1.t().contiguous(), f), C2)
+
+
+def exact(case, seed):
+    kind, n = case["kind"], _size(case)
+    if kind == "poisson":
+        length, eps, source, volts = _poisson_inputs(case, seed)
+        h = [L / m for L, m in zip(length, n)]
+        d = eps[:, 0, 0]
+        w = torch.zeros(n[2] + 1, dtype=F64, device=DEV)
+        w[1:-1] = 0.5 * (d[:-1] + d[1:]) / h[2] ** 2
+        w[0], w[-1] = 2 * d[0] / h[2] ** 2, 2 * d[-1] / h[2] ** 2
+        rhs = source.clone()
+        rhs[-1] += w[-1] * volts
+        return _separable(-w[:-1], w[:-1] + w[1:], -w[1:], d, (h[1], h[0]), rhs)
+    if kind == "cdr":
+        length, base, old = _cdr_inputs(case, seed)
+        h = [L / m for L, m in zip(length, n)]
+        one = torch.ones(n[0], dtype=F64, device=DEV)
+        w, v = 0.5 / h[0] ** 2, 1.0 / h[0]
+        diag = (2 * w + v - 2.0 + 10.0) * one
+        diag[0] += w            # the wall's half cell
+        diag[-1] -= w
+        rhs = base + 10.0 * old
+        rhs[:, :, -1] += 0.25 / h[0]
+        u = _separable(-w * one, diag, -(w + v) * one, 0.5 * one, (h[2], h[1]), rhs.permute(2, 0, 1).contiguous())
+        return u.permute(1, 2, 0).contiguous()
+    return None
