@@ -269,6 +269,7 @@ def run(state):
     if kind in ("glow", "five"):
         with torch.no_grad():
             dens, neps = state["model"].step(state["dens"], state["neps"], state["V"])
+        state["dens"], state["neps"] = dens, neps   # the next pass is the next step
         return {"dens": list(dens), "neps": neps, "phi": state["model"]._phi}
     if kind == "plasma":
         r = state["run"]
