@@ -839,6 +839,30 @@ double *bottom_work<double>(mps_ctx *c) { return c->bottom64; }
 template <>
 float *bottom_work<float>(mps_ctx *c) { return c->bottom32; }
 
+// performgmres with GMRES(m) on a level: one wavefront (k_bottom_wave) for at
+// most kWaveN cells and m, where a lane per cell holds the whole problem
+// (64 cells, 64 Arnoldi steps: BOTTOM_FIG); else, and for rows
+// in fast arithmetic (whose contracted sums only row7 forms), k_bottom with
+// the Hessenberg matrix in LDS for m <= kBottomLdsM
+template <typename T>
+void launch_ref_gmres(mps_ctx *c, const Lev<T> &v, T *u, const T *b, T *work, int op, int m, int nrestarts, T tol)
+{
+    const long long n = (long long)v.nx * v.ny * v.nz;
+    with_op(op, c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
+        constexpr int OPC = decltype(O)::value;
+        constexpr bool VC = decltype(V)::value, RC = decltype(R)::value;
+        if (n <= kWaveN && m <= kWaveN && (OPC == OP_STENCIL || !v.fast))
+            hipLaunchKernelGGL((k_bottom_wave<T, OPC, VC, RC>), dim3(1), dim3(kWaveN), 0, c->stream, v, u, b, m,
+                               nrestarts, tol, c->d_status);
+        else if (m <= kBottomLdsM)
+            hipLaunchKernelGGL((k_bottom<T, OPC, VC, RC, true>), dim3(1), block(), 0, c->stream, v, u, b, work, m,
+                               nrestarts, tol, c->d_status);
+        else
+            hipLaunchKernelGGL((k_bottom<T, OPC, VC, RC, false>), dim3(1), block(), 0, c->stream, v, u, b, work, m,
+                               nrestarts, tol, c->d_status);
+    });
+}
+
 template <typename T>
 void launch_bottom(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, int op, T *work)
 {
@@ -849,18 +873,7 @@ void launch_bottom(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, int op, T *wo
     }
     // err_tol = ERRTOLR*0.0001 with a default-real literal (mgridsteps.f90:305)
     const T tol = (T)(1e-11 * (double)0.0001f);
-    const int m = (int)c->geom[l].n();
-    const dim3 bb = block();
-    with_op(op, c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
-        if (m <= kBottomLdsM)
-            hipLaunchKernelGGL((k_bottom<T, decltype(O)::value, decltype(V)::value, decltype(R)::value, true>),
-                               dim3(1), bb, 0, c->stream, v, L[l].u, (const T *)L[l].b, work, m, 1, tol,
-                               c->d_status);
-        else
-            hipLaunchKernelGGL((k_bottom<T, decltype(O)::value, decltype(V)::value, decltype(R)::value, false>),
-                               dim3(1), block(), 0, c->stream, v, L[l].u, (const T *)L[l].b, work, m, 1, tol,
-                               c->d_status);
-    });
+    launch_ref_gmres<T>(c, v, L[l].u, (const T *)L[l].b, work, op, (int)c->geom[l].n(), 1, tol);
 }
 
 // fused red-black sweep u -> u2 (see mps3d_sweep.h)
@@ -3381,16 +3394,7 @@ void gmres_ref_launch(mps_ctx *c, const double *bd, double *u, int m, int max_re
     fill<double>(c, bg, g.ng(), 0.0);
     Lev<double> v = view(c, c->L64, 0);
     hipLaunchKernelGGL(k_interior_in<double>, cells_grid(g), block(), 0, c->stream, v, bd, bg);
-    with_op(level_op(c, 0), c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
-        if (m <= kBottomLdsM)
-            hipLaunchKernelGGL((k_bottom<double, decltype(O)::value, decltype(V)::value, decltype(R)::value, true>),
-                               dim3(1), block(), 0, c->stream, v, u, (const double *)bg, work, m, max_restarts, tol,
-                               c->d_status);
-        else
-            hipLaunchKernelGGL((k_bottom<double, decltype(O)::value, decltype(V)::value, decltype(R)::value, false>),
-                               dim3(1), block(), 0, c->stream, v, u, (const double *)bg, work, m, max_restarts, tol,
-                               c->d_status);
-    });
+    launch_ref_gmres<double>(c, v, u, (const double *)bg, work, level_op(c, 0), m, max_restarts, tol);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(c->h_scalar + 1, c->d_status, sizeof(int), hipMemcpyDeviceToHost, c->stream));
 }

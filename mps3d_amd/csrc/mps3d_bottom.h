@@ -357,6 +357,385 @@ __global__ void __launch_bounds__(kBlock) k_bottom(Lev<T> L, T *u, const T *__re
 }
 
 // ------------------------------------------------------------------------
+// The same solve for at most kWaveN cells and m <= kWaveN in one wavefront,
+// bit for bit k_bottom's result. Lane q owns cell q; the level's row of that
+// cell (diagonal, face conductances, face velocities) stays in registers
+// for the whole solve, the Krylov basis, the Hessenberg matrix and the
+// vectors that other lanes read stay in LDS, and nothing waits on global
+// memory or on a workgroup barrier between the first load and the last
+// store. What bounds it is the instruction count of one wave (4 cycles each)
+// on the reference's serial summation order: an Arnoldi step is two chains
+// of n dependent additions (the kd Gram-Schmidt products, one per lane, and
+// the norm) and one of kd subtractions. Those loops are laid out flat in
+// chunks that a uniform branch skips, with the next chunk's LDS loads ahead
+// of the additions. Two things that the reference does step by step on
+// one value at a time are done once, in another loop order with the same
+// operands and results: the Givens rotations of all columns after the last
+// Arnoldi step (the iteration reads none of them), one column per lane, and
+// the products of the back substitution's rows.
+// Sums run over whole chunks: the entries past n (or past kd) are zero, and
+// adding or subtracting +0 leaves every partial sum as it is (a sum that
+// starts at +0 is never -0). 64 cells, 64 steps: 148 us, of it 110 us in the
+// Arnoldi steps (4200 cycles each: products 1230, subtractions 1020, norm
+// 840, operator and preconditioner 830), rotations 15 us, back substitution
+// 22 us; with rolled loops and broadcasts through ds_bpermute 204 us.
+// ------------------------------------------------------------------------
+constexpr int kWaveN = 64;            // one cell per lane
+constexpr int kWaveLd = kWaveN + 2;   // entries kWaveN, kWaveN + 1 of a row stay zero
+
+template <typename T>
+struct alignas(2 * sizeof(T)) PairT {
+    T a, b;
+};
+
+// LDS operations of one wave complete in order: between a lane's write and
+// another lane's read only the compiler has to be held
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// the value of lane q (uniform)
+__device__ __forceinline__ double lane_value(double v, int q)
+{
+    const long long b = __builtin_bit_cast(long long, v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)b, q), hi = __builtin_amdgcn_readlane((int)(b >> 32), q);
+    return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ float lane_value(float v, int q)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), q));
+}
+
+// s + a[0] c[0] + a[1] c[1] + ... (FORM 1), s + a[0] + a[1] + ... (FORM 0) or
+// s - a[0] - a[1] - ... (FORM -1), n terms in order, in chunks of 16 (a, c
+// aligned to a pair, zero past n up to the next chunk)
+template <typename T, int FORM>
+__device__ __forceinline__ T serial_sum(T s, const T *a, const T *c, int n)
+{
+    constexpr int K = 8, NC = kWaveN / (2 * K);
+    const PairT<T> *pa = reinterpret_cast<const PairT<T> *>(a);
+    const PairT<T> *pc = reinterpret_cast<const PairT<T> *>(c);
+    PairT<T> ra[NC][K], rc[NC][K];
+    auto load = [&](int g) {
+#pragma unroll
+        for (int t = 0; t < K; ++t) {
+            ra[g][t] = pa[g * K + t];
+            if (FORM == 1) rc[g][t] = pc[g * K + t];
+        }
+    };
+    auto add = [&](int g) {
+#pragma unroll
+        for (int t = 0; t < K; ++t) {
+            if (FORM == -1) {
+                s = s - ra[g][t].a;
+                s = s - ra[g][t].b;
+            } else {
+                s = s + (FORM == 1 ? ra[g][t].a * rc[g][t].a : ra[g][t].a);
+                s = s + (FORM == 1 ? ra[g][t].b * rc[g][t].b : ra[g][t].b);
+            }
+        }
+    };
+    load(0);
+    if (n > 16) {
+        load(1);
+        add(0);
+        if (n > 32) {
+            load(2);
+            add(1);
+            if (n > 48) {
+                load(3);
+                add(2);
+                add(3);
+            } else {
+                add(2);
+            }
+        } else {
+            add(1);
+        }
+    } else {
+        add(0);
+    }
+    return s;
+}
+
+// t - h[0] V[0][lane] - h[1] V[1][lane] - ... in that order, kd terms in
+// chunks of 8 (h zero past kd, V finite)
+template <typename T, int G = 0>
+__device__ __forceinline__ T serial_axpy(T t, const T *h, const T (*V)[kWaveLd], int lane, int kd, const PairT<T> *h0,
+                                         const T *v0)
+{
+    constexpr int K = 8;
+    PairT<T> h1[K / 2];
+    T v1[K];
+    if constexpr (8 * (G + 1) < kWaveN) {
+        const PairT<T> *ph = reinterpret_cast<const PairT<T> *>(h) + K / 2 * (G + 1);
+#pragma unroll
+        for (int p = 0; p < K / 2; ++p) h1[p] = ph[p];
+#pragma unroll
+        for (int p = 0; p < K; ++p) v1[p] = V[K * (G + 1) + p][lane];
+    }
+#pragma unroll
+    for (int p = 0; p < K / 2; ++p) {
+        t = t - h0[p].a * v0[2 * p];
+        t = t - h0[p].b * v0[2 * p + 1];
+    }
+    if constexpr (8 * (G + 1) < kWaveN) {
+        if (kd > 8 * (G + 1)) return serial_axpy<T, G + 1>(t, h, V, lane, kd, h1, v1);
+    }
+    return t;
+}
+
+template <typename T, int OP, bool VEL, bool REAC>
+__global__ void __launch_bounds__(kWaveN) k_bottom_wave(Lev<T> L, T *u, const T *__restrict__ b, int m, int nrestarts,
+                                                       T tol, int *status)
+{
+    // basis vectors by row, Hessenberg columns by row (entry ii of column kd
+    // at sH[kd][ii], 0-based)
+    __shared__ alignas(16) T sV[kWaveN + 1][kWaveLd];
+    __shared__ alignas(16) T sH[kWaveN][kWaveLd];
+    __shared__ alignas(16) T sr[kWaveLd];   // red values of the preconditioner
+    __shared__ alignas(16) T sw[kWaveLd];   // the vector or products that every lane reads
+    const int lane = threadIdx.x;
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
+    const int n = nx * ny * nz;
+    const bool own = lane < n;
+    const int q0 = own ? lane : 0;
+    const int i = q0 % nx + 1, j = (q0 / nx) % ny + 1, k = q0 / (nx * ny) + 1;
+    const long long c = (long long)i + (long long)L.sy * j + L.sz * k;
+    const bool red = ((i + j + k) & 1) == 1;
+    // the six neighbours in a row of sV, sr: kWaveN (a zero) where the face
+    // does not exist
+    const bool ex[6] = {i > 1, i < nx, j > 1, j < ny, k > 1, k < nz};
+    const int nb[6] = {ex[0] ? lane - 1 : kWaveN,       ex[1] ? lane + 1 : kWaveN,  ex[2] ? lane - nx : kWaveN,
+                       ex[3] ? lane + nx : kWaveN,      ex[4] ? lane - nx * ny : kWaveN,
+                       ex[5] ? lane + nx * ny : kWaveN};
+    // The row. face_right and face_left add 0 - u kq ab and, on the upwind
+    // side, -+ vh u ab per face (kq = kh / d): a face's two multipliers of
+    // u carry those signs, and a term that does not exist has multiplier 0
+    // (its +-0 leaves the sum as it is). Explicit rows: kq = st.
+    T dg, kq[6], vq[6], ab[3];
+    const T bc = own ? b[c] : T(0);
+    T x = own ? u[c] : T(0);
+    {
+        // (every load first: the ghosted arrays hold every neighbour, so no
+        // load waits on a test of the face before it)
+        const long long st[3] = {1, L.sy, L.sz};
+        const T *v3[3] = {L.vx, L.vy, L.vz};
+        const T h[3] = {L.dx, L.dy, L.dz};
+        const T a0[3] = {L.ax, L.ay, L.az}, a1[3] = {L.axb, L.ayb, L.azb}, i0[3] = {L.ix0, L.iy0, L.iz0};
+        T Dn[6], vn[6], vc[3], Dc = T(0), rc = T(0);
+#pragma unroll
+        for (int f = 0; f < 6; ++f) {
+            const long long o = (f & 1) ? c + st[f / 2] : c - st[f / 2];
+            if (OP == OP_STENCIL) kq[f] = L.st[1 + f][c];
+            else Dn[f] = L.D[o];
+            if (VEL) vn[f] = v3[f / 2][o];
+            if (VEL && !(f & 1)) vc[f / 2] = v3[f / 2][c];
+        }
+        if (OP == OP_STENCIL) dg = L.st[ST_C][c];
+        else Dc = L.D[c];
+        if (OP != OP_STENCIL && REAC) rc = L.reac[c];
+        if (OP != OP_STENCIL) {
+            // the diagonal in row()'s order: per direction the two faces,
+            // then the wall terms; reaction and time last
+            T d = T(0);
+#pragma unroll
+            for (int f = 0; f < 6; ++f) {
+                const int q = f / 2;
+                const bool edge = !ex[2 * q] || !ex[2 * q + 1];
+                ab[q] = (OP == OP_ALIGNED && edge) ? a1[q] : a0[q];
+                // (left + right, in that order, as the face functions add)
+                const T kf = (T(0.5) * ((f & 1) ? Dc + Dn[f] : Dn[f] + Dc)) / h[q];
+                T t = T(0) + kf * ab[q];
+                kq[f] = ex[f] ? -kf : T(0);
+                if (VEL) {
+                    const T vh = T(0.5) * ((f & 1) ? vc[q] + vn[f] : vn[f] + vc[q]);
+                    const bool pos = vh > T(0);
+                    // the upwind cell of the face is the left one where vh > 0
+                    if (f & 1) t = pos ? t + vh * ab[q] : t;
+                    else t = pos ? t : t - vh * ab[q];
+                    vq[f] = (ex[f] && pos == !(f & 1)) ? ((f & 1) ? vh : -vh) : T(0);
+                }
+                if (ex[f]) d = d + t;
+                if (f & 1) {
+                    if (!ex[f - 1])
+                        bc_row<T, OP, VEL>(L.bc[f - 1], false, Dc, VEL ? vc[q] : T(0), h[q], ab[q], i0[q], d);
+                    if (!ex[f]) bc_row<T, OP, VEL>(L.bc[f], true, Dc, VEL ? vc[q] : T(0), h[q], ab[q], i0[q], d);
+                }
+            }
+            if (REAC) d = d - rc;
+            if (L.timederiv) d = d + T(1) / L.dt;
+            dg = d;
+        }
+    }
+    // off-diagonal sum of this lane's row over neighbour values in a row of LDS
+    auto offdiag = [&](const T *p) {
+        T un[6];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) un[f] = p[nb[f]];
+        T o = T(0);
+#pragma unroll
+        for (int f = 0; f < 6; ++f) {
+            if (OP == OP_STENCIL) {
+                o = o + kq[f] * un[f];
+            } else {
+                T t = un[f] * kq[f] * ab[f / 2];
+                if (VEL) t = t + vq[f] * un[f] * ab[f / 2];
+                o = o + t;
+            }
+        }
+        return o;
+    };
+    sr[lane] = T(0);
+    for (int q = 0; q <= kWaveN; ++q) sV[q][lane] = T(0);
+    sV[lane][kWaveN] = sV[lane][kWaveN + 1] = T(0);
+    if (lane < 2) sr[kWaveN + lane] = T(0), sw[kWaveN + lane] = T(0);
+    wave_fence();
+    const T of0 = offdiag(sr);   // of a red cell: its black neighbours are cleared
+    // gseidel_precond of the vector whose entry of this cell is `in`
+    auto precond = [&](T in) {
+        T v = (in - of0) / dg;
+        sr[lane] = (own && red) ? v : T(0);
+        wave_fence();
+        const T o = offdiag(sr);
+        if (!red) v = (in - o) / dg;
+        wave_fence();
+        return own ? v : T(0);
+    };
+    auto norm = [&](T v) {
+        sw[lane] = v * v;
+        wave_fence();
+        const T s = serial_sum<T, 0>(T(0), sw, sw, n);
+        wave_fence();
+        return sqrt(s);
+    };
+
+    if (lane == 0) *status = 0;
+    for (int rs = 1; rs <= nrestarts; ++rs) {
+        const T bnorm = norm(precond(bc));
+        if (bnorm == T(0)) {
+            x = T(0);
+            break;
+        }
+        const T x0 = x;
+        sw[lane] = x0;
+        wave_fence();
+        const T av0 = dg * x0 + offdiag(sw);
+        wave_fence();
+        const T r = precond(own ? bc - av0 : T(0));
+        const T beta = norm(r);
+        if (fabs((double)beta) < (double)tol) break;
+        T v = own ? r / beta : T(0);   // the newest basis vector's entry
+        sV[0][lane] = v;
+        wave_fence();
+        int optk = m, lucky = 0;
+        for (int kd = 1; kd <= m; ++kd) {
+            const T av = dg * v + offdiag(sV[kd - 1]);
+            const T w = precond(own ? av : T(0));
+            sw[lane] = w;
+            wave_fence();
+            // h_ii = <w, v_ii>, lane ii - 1 (of the rows filled so far)
+            T *hk = sH[kd - 1];
+            const T h = serial_sum<T, 1>(T(0), sw, sV[lane], n);
+            hk[lane] = lane < kd ? h : T(0);
+            wave_fence();
+            // w - h_1 v_1 - h_2 v_2 - ... in that order
+            PairT<T> h0[4];
+            T v0[8];
+#pragma unroll
+            for (int p = 0; p < 8; ++p) v0[p] = sV[p][lane];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) h0[p] = reinterpret_cast<const PairT<T> *>(hk)[p];
+            const T t = serial_axpy<T>(w, hk, sV, lane, kd, h0, v0);
+            const T hn = norm(t);
+            if (hn > T(1e-25)) {
+                v = own ? t / hn : T(0);
+                sV[kd][lane] = v;
+            } else if (!(hn != hn) && !((hn / hn != T(1)) && hn != T(0))) {
+                lucky = 1;
+            } else {
+                if (lane == 0) *status = -1;
+                return;
+            }
+            if (lane == 0) hk[kd] = hn;
+            wave_fence();
+            if (lucky) {
+                optk = kd;
+                break;
+            }
+        }
+        // triangularize (gmres.f90:159-195): rotation ii is formed from
+        // column ii and applied to the columns after it, lane = column; hc is
+        // the column's entry of row ii after the rotations before
+        T bl = T(0), bcur = beta;   // be(ii) of lane ii, be(ii + 1) so far
+        T rdiag = T(1), rsup = T(0);   // R(lane, lane), R(lane - 1, lane)
+        {
+            T *const col = sH[min(lane, optk - 1)];
+            T hc = col[0], hn1 = col[1];
+            for (int ii = 0; ii < optk; ++ii) {
+                const T hn2 = col[min(ii + 2, kWaveN)];
+                const T rr = lane_value(hc, ii), ss = lane_value(hn1, ii);
+                T cs, sn;
+                if (rr == T(0)) {
+                    cs = T(0);
+                    sn = T(1);
+                } else {
+                    const T den = sqrt(rr * rr + ss * ss);
+                    cs = rr / den;
+                    sn = ss / den;
+                }
+                const T t = cs * hc + sn * hn1;
+                hc = -sn * hc + cs * hn1;
+                hn1 = hn2;
+                if (lane == ii) {
+                    rdiag = t;
+                    bl = cs * bcur;
+                }
+                if (lane == ii + 1) rsup = t;
+                if (lane > ii && lane < optk) col[ii] = t;
+                bcur = -sn * bcur;
+            }
+        }
+        const T residnorm = fabs(bcur);
+        wave_fence();
+        // uppertrisolve (gmres.f90:124-142): row ii subtracts its products
+        // in ascending columns. Those of the columns past ii + 1 are formed
+        // (lane = column) and stored a row ahead, so that only y(ii + 1)'s
+        // own is formed when it is known; the sum runs over whole chunks of
+        // 16 (zeros before column ii + 2 and past optk)
+        T y = T(0), yi = T(0);
+        sw[lane] = T(0);
+        T hrow = sH[lane][max(optk - 2, 0)];   // R(ii - 1, lane) at row ii
+        wave_fence();
+        for (int ii = optk - 1; ii >= 0; --ii) {
+            T s = lane_value(bl, ii);
+            if (ii + 1 < optk) {
+                s = s - lane_value(rsup, ii + 1) * yi;
+                const int j0 = (ii + 2) & ~15;
+                if (j0 < optk) s = serial_sum<T, -1>(s, sw + j0, sw, optk - j0);
+            }
+            wave_fence();
+            sw[lane] = (lane > ii && lane < optk) ? hrow * y : T(0);
+            hrow = sH[lane][max(ii - 2, 0)];
+            yi = s / lane_value(rdiag, ii);
+            if (lane == ii) y = yi;
+            wave_fence();
+        }
+        sw[lane] = y;
+        wave_fence();
+        T xv = x0;
+#pragma unroll 8
+        for (int jj = 0; jj < optk; ++jj) xv = xv + sw[jj] * sV[jj][lane];
+        x = xv;
+        wave_fence();
+        if (residnorm / bnorm <= tol || lucky) break;
+    }
+    if (own) u[c] = x;
+}
+
+// ------------------------------------------------------------------------
 // Scharfetter-Gummel operator rows
 // ------------------------------------------------------------------------
 
