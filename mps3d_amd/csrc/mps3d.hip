@@ -195,6 +195,8 @@ struct mps_ctx {
     double *user_tmp2 = nullptr;         // staging for interior arrays
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t ev_in = nullptr;          // orders calls after the null stream
+    hipEvent_t ev_inv = nullptr;         // the coarsest inverse's status has been copied
+    bool inv_pending = false;            // and set_coeffs has yet to read it
     double last_ms = 0.0;
     int last_cycles = 0;
     double *dinv = nullptr;              // dense inverse of the coarsest operator
@@ -541,6 +543,17 @@ void fill(mps_ctx *c, T *p, long long n, T v)
 {
     long long blocks = std::min<long long>((n + kBlock - 1) / kBlock, 65536);
     hipLaunchKernelGGL(k_fill<T>, dim3((unsigned)std::max<long long>(blocks, 1)), block(), 0, c->stream, p, n, v);
+}
+
+// an array of n zeros on first use, kept as it is afterwards
+template <typename T>
+T *zeroed(mps_ctx *c, T *&p, long long n)
+{
+    if (!p) {
+        p = dalloc<T>(n);
+        fill<T>(c, p, n, T(0));
+    }
+    return p;
 }
 
 template <typename Ti, typename To>
@@ -1272,11 +1285,14 @@ void derive_coarse(mps_ctx *c)
             hipLaunchKernelGGL(k_restrict_mean5, cells_grid(gc), block(), 0, c->stream, vf, vc, F);
         } else {
             AlignedW W{L[l].w[0], L[l].w[1], L[l].w[2]};
+            dim3 gr = cells_grid(gc);
+            gr.z = 0;
             for (int q = 0; q < 5; ++q) {
                 if (!F.src[q]) continue;
-                hipLaunchKernelGGL(k_restrict_fw<double>, cells_grid(gc), block(), 0, c->stream, vf, vc, W,
-                                   (const double *)F.src[q], F.dst[q]);
+                F.src[gr.z] = F.src[q];
+                F.dst[gr.z++] = F.dst[q];
             }
+            hipLaunchKernelGGL(k_restrict_fw5, gr, block(), 0, c->stream, vf, vc, W, F);
         }
     }
 }
@@ -1325,16 +1341,10 @@ void conductance_coarse_levels(mps_ctx *c)
                                W, (const double *)f[3 * l - 3], (const double *)f[3 * l - 2],
                                (const double *)f[3 * l - 1], f[3 * l], f[3 * l + 1], f[3 * l + 2]);
             LevelBuf<double> &B = L[l];
-            for (int q = 0; q < ST_N; ++q) {
-                if (!B.st[q]) B.st[q] = dalloc<double>(g.ng());
-                fill<double>(c, B.st[q], g.ng(), 0.0);
-            }
+            for (int q = 0; q < ST_N; ++q) zeroed<double>(c, B.st[q], g.ng());
             // face form: conductances (ghost entries stay 0: the boundary
             // faces) and the diagonal of st
-            for (int q = 1; q < 4; ++q) {
-                if (!B.fc[q]) B.fc[q] = dalloc<double>(g.ng());
-                fill<double>(c, B.fc[q], g.ng(), 0.0);
-            }
+            for (int q = 1; q < 4; ++q) zeroed<double>(c, B.fc[q], g.ng());
             B.fc[0] = B.st[ST_C];
             hipLaunchKernelGGL(k_faces_stencil, cells_grid(g), block(), 0, c->stream, view(c, L, l),
                                (const double *)f[3 * l], (const double *)f[3 * l + 1], (const double *)f[3 * l + 2],
@@ -1349,34 +1359,33 @@ void conductance_coarse_levels(mps_ctx *c)
     for (auto p : f) dfree(p);
 }
 
-void build_stencils(mps_ctx *c, std::vector<LevelBuf<double>> &L, bool transpose)
+// explicit rows of level l (the forward hierarchy's, with the FP32 cycle's
+// copy of Scharfetter-Gummel rows, or the transposed one's)
+void build_stencil(mps_ctx *c, std::vector<LevelBuf<double>> &L, int l, bool transpose)
 {
-    for (int l = 0; l < c->nlev(); ++l) {
-        const Geom &g = c->geom[l];
-        LevelBuf<double> &B = L[l];
-        for (int q = 0; q < ST_N; ++q) {
-            if (!B.st[q]) B.st[q] = dalloc<double>(g.ng());
-            fill<double>(c, B.st[q], g.ng(), 0.0);
-        }
-        // coefficient views come from the FP64 forward hierarchy
-        Lev<double> v = view(c, c->L64, l);
-        const bool aligned = c->opts.hierarchy == MPS_HIER_ALIGNED && l > 0;
-        if (c->opts.flux == MPS_FLUX_SG) {
-            if (aligned)
-                hipLaunchKernelGGL(k_sg_stencil<OP_ALIGNED>, cells_grid(g), block(), 0, c->stream, v, B.st[0],
-                                   B.st[1], B.st[2], B.st[3], B.st[4], B.st[5], B.st[6], transpose ? 1 : 0);
-            else
-                hipLaunchKernelGGL(k_sg_stencil<OP_REF>, cells_grid(g), block(), 0, c->stream, v, B.st[0], B.st[1],
-                                   B.st[2], B.st[3], B.st[4], B.st[5], B.st[6], transpose ? 1 : 0);
-        } else {
-            const int op = aligned ? OP_ALIGNED : OP_REF;
-            with_op(op, c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
-                hipLaunchKernelGGL((k_build_stencil<double, decltype(O)::value, decltype(V)::value,
-                                                    decltype(R)::value>),
-                                   cells_grid(g), block(), 0, c->stream, v, B.st[0], B.st[1], B.st[2], B.st[3],
-                                   B.st[4], B.st[5], B.st[6], transpose ? 1 : 0);
-            });
-        }
+    const Geom &g = c->geom[l];
+    LevelBuf<double> &B = L[l];
+    // (the kernels write the same interior entries on every call: what they
+    // leave out stays zero from the allocation on)
+    RowArrays S{};
+    for (int q = 0; q < ST_N; ++q) S.st[q] = zeroed<double>(c, B.st[q], g.ng());
+    // coefficient views come from the FP64 forward hierarchy
+    Lev<double> v = view(c, c->L64, l);
+    const bool aligned = c->opts.hierarchy == MPS_HIER_ALIGNED && l > 0;
+    if (c->opts.flux == MPS_FLUX_SG) {
+        if (!transpose && c->opts.precision == MPS_PREC_FP32_DC)
+            for (int q = 0; q < ST_N; ++q) S.st32[q] = zeroed<float>(c, c->L32[l].st[q], g.ng());
+        if (aligned)
+            hipLaunchKernelGGL(k_sg_stencil<OP_ALIGNED>, cells_grid(g), block(), 0, c->stream, v, S, transpose ? 1 : 0);
+        else
+            hipLaunchKernelGGL(k_sg_stencil<OP_REF>, cells_grid(g), block(), 0, c->stream, v, S, transpose ? 1 : 0);
+    } else {
+        const int op = aligned ? OP_ALIGNED : OP_REF;
+        with_op(op, c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
+            hipLaunchKernelGGL((k_build_stencil<double, decltype(O)::value, decltype(V)::value, decltype(R)::value>),
+                               cells_grid(g), block(), 0, c->stream, v, B.st[0], B.st[1], B.st[2], B.st[3], B.st[4],
+                               B.st[5], B.st[6], transpose ? 1 : 0);
+        });
     }
 }
 
@@ -1387,15 +1396,19 @@ void build_fp32(mps_ctx *c)
     auto &F = c->L32;
     for (int l = 0; l < c->nlev(); ++l) {
         const long long ng = c->geom[l].ng();
-        convert<double, float>(c, L[l].D, F[l].D, ng);
-        double *src[4] = {L[l].vx, L[l].vy, L[l].vz, L[l].reac};
-        float **dst[4] = {&F[l].vx, &F[l].vy, &F[l].vz, &F[l].reac};
-        for (int q = 0; q < 4; ++q) {
-            if (!src[q]) continue;
-            if (!*dst[q]) *dst[q] = dalloc<float>(ng);
-            convert<double, float>(c, src[q], *dst[q], ng);
+        // (a level of explicit rows reads no cell coefficients; its
+        // Scharfetter-Gummel rows were written in FP32 with the FP64 ones)
+        if (level_op(c, F, l) != OP_STENCIL) {
+            convert<double, float>(c, L[l].D, F[l].D, ng);
+            double *src[4] = {L[l].vx, L[l].vy, L[l].vz, L[l].reac};
+            float **dst[4] = {&F[l].vx, &F[l].vy, &F[l].vz, &F[l].reac};
+            for (int q = 0; q < 4; ++q) {
+                if (!src[q]) continue;
+                if (!*dst[q]) *dst[q] = dalloc<float>(ng);
+                convert<double, float>(c, src[q], *dst[q], ng);
+            }
         }
-        for (int q = 0; q < ST_N; ++q) {
+        for (int q = 0; q < ST_N && c->opts.flux != MPS_FLUX_SG; ++q) {
             if (!L[l].st[q]) continue;
             if (!F[l].st[q]) F[l].st[q] = dalloc<float>(ng);
             convert<double, float>(c, L[l].st[q], F[l].st[q], ng);
@@ -1795,81 +1808,101 @@ int solve_core(mps_ctx *c, double *u, double *b, bool homog, double *history, do
     return it;
 }
 
-// coarsest-level dense inverse for the aligned hierarchy: assembles the
-// coarsest operator from its 7-point rows and inverts it (Gauss-Jordan with
-// partial pivoting, FP64) once per set of coefficients
-// Reference hierarchy in fast arithmetic: the coarsest operator's inverse
-// built on the device (k_dense_inverse) once per set of coefficients; the
-// V-cycle's coarse GMRES becomes one matrix-vector product.
-void build_bottom_inverse_device(mps_ctx *c)
+// The coarsest operator's dense inverse on the device: queued by
+// launch_bottom_inverse as soon as that level's rows are (or its
+// coefficients), once per set of coefficients. Coarsest grids of more than
+// kInvRegsN cells: on the reference hierarchy the kernel with the matrix in
+// global memory, on the aligned hierarchy host_bottom_inverse.
+// The aligned hierarchy refuses a singular coarsest operator: the kernel's
+// verdict is copied to pinned memory behind an event, which
+// finish_bottom_inverse waits for while the finer levels' set-up runs.
+int bottom_rows(mps_ctx *c, RowArrays &S)
 {
     const int lb = c->nlev() - 1;
     const Geom &g = c->geom[lb];
-    const int n = (int)g.n();
-    if (n > kBottomMaxDense) return;   // k_bottom stays
-    const long long ng = g.ng();
-    for (int q = 0; q < ST_N; ++q)
-        if (!c->bst[q]) {
-            c->bst[q] = dalloc<double>(ng);
-            fill<double>(c, c->bst[q], ng, 0.0);
-        }
-    if (!c->dinv) c->dinv = dalloc<double>((size_t)kBottomMaxDense * kBottomMaxDense);
-    if (n > kDenseLdsN && !c->dwork) c->dwork = dalloc<double>((size_t)kBottomMaxDense * kBottomMaxDense);
+    const bool aligned = c->opts.hierarchy == MPS_HIER_ALIGNED;
+    if (aligned && level_op(c, c->L64, lb) == OP_STENCIL) {
+        for (int q = 0; q < ST_N; ++q) S.st[q] = c->L64[lb].st[q];
+        return lb;
+    }
+    for (int q = 0; q < ST_N; ++q) S.st[q] = zeroed<double>(c, c->bst[q], g.ng());
     Lev<double> v = view(c, c->L64, lb);
     with_op(level_op(c, lb), c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
         hipLaunchKernelGGL((k_build_stencil<double, decltype(O)::value, decltype(V)::value, decltype(R)::value>),
-                           cells_grid(g), block(), 0, c->stream, v, c->bst[0], c->bst[1], c->bst[2], c->bst[3],
-                           c->bst[4], c->bst[5], c->bst[6], 0);
+                           cells_grid(g), block(), 0, c->stream, v, S.st[0], S.st[1], S.st[2], S.st[3], S.st[4],
+                           S.st[5], S.st[6], 0);
     });
-#ifndef MPS_DENSE_LDS_THREADS
-#define MPS_DENSE_LDS_THREADS 1024
-#endif
-    const unsigned nth = n <= kDenseLdsN ? MPS_DENSE_LDS_THREADS : kDenseThreads;
-    hipLaunchKernelGGL(k_dense_inverse, dim3(1), dim3(nth), 0, c->stream, v, (const double *)c->bst[0],
-                       (const double *)c->bst[1], (const double *)c->bst[2], (const double *)c->bst[3],
-                       (const double *)c->bst[4], (const double *)c->bst[5], (const double *)c->bst[6], c->dwork,
-                       c->dinv, (int *)nullptr);
+    return lb;
+}
+
+void launch_bottom_inverse(mps_ctx *c)
+{
+    for (auto &B : c->L64) B.inv = nullptr;
+    for (auto &B : c->L32) B.inv = nullptr;
+    c->inv_pending = false;
+    const bool aligned = c->opts.hierarchy == MPS_HIER_ALIGNED;
+    if (!c->mg_ok || (!aligned && c->opts.arith != MPS_ARITH_FAST)) return;
+    const long long n = c->geom.back().n();
+    if (n > kBottomMaxDense) {
+        if (aligned) throw HipError{hipErrorInvalidValue, "coarsest grid too large for a dense solve"};
+        return;   // the reference GMRES stays
+    }
+    if (aligned && n > kInvRegsN) return;   // host_bottom_inverse
+    const size_t full = (size_t)kBottomMaxDense * kBottomMaxDense;
+    if (!c->dinv) c->dinv = dalloc<double>(full);
+    if (aligned && !c->dinvT) c->dinvT = dalloc<double>(full);
+    RowArrays S{};
+    const int lb = bottom_rows(c, S);
+    Lev<double> v = view(c, c->L64, lb);
+    double *invT = aligned ? c->dinvT : nullptr;
+    int *st = aligned ? c->d_status + 1 : nullptr;
+    auto go = [&](auto E) {
+        hipLaunchKernelGGL((k_dense_inverse_regs<decltype(E)::value>), dim3(1), dim3(kInvThreads), 0, c->stream, v, S,
+                           c->dinv, invT, st);
+    };
+    if (n <= 32) go(IntC<1>{});
+    else if (n <= 64) go(IntC<2>{});
+    else if (n <= 128) go(IntC<4>{});
+    else if (n <= kInvRegsN) go(IntC<7>{});
+    else {
+        if (!c->dwork) c->dwork = dalloc<double>(full);
+        hipLaunchKernelGGL(k_dense_inverse, dim3(1), dim3(kDenseThreads), 0, c->stream, v, S, c->dwork, c->dinv);
+    }
     HIPCHK(hipGetLastError());
+    if (aligned) {
+        HIPCHK(hipMemcpyAsync(c->h_scalar + 2, st, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipEventRecord(c->ev_inv, c->stream));
+        c->inv_pending = true;
+    }
     c->L64[lb].inv = c->dinv;
     if (!c->L32.empty()) c->L32[lb].inv = c->dinv;
 }
 
-void build_bottom_inverse(mps_ctx *c)
+void finish_bottom_inverse(mps_ctx *c)
 {
+    if (!c->inv_pending) return;
+    c->inv_pending = false;
+    HIPCHK(hipEventSynchronize(c->ev_inv));
+    int st;
+    std::memcpy(&st, c->h_scalar + 2, sizeof(int));
+    if (st == 0) return;
     for (auto &B : c->L64) B.inv = nullptr;
     for (auto &B : c->L32) B.inv = nullptr;
-    if (c->mg_ok && c->opts.hierarchy == MPS_HIER_REF && c->opts.arith == MPS_ARITH_FAST) {
-        build_bottom_inverse_device(c);
-        return;
-    }
-    if (!c->mg_ok || c->opts.hierarchy != MPS_HIER_ALIGNED) return;
+    throw HipError{hipErrorInvalidValue, "singular coarsest-level operator"};
+}
+
+void host_bottom_inverse(mps_ctx *c)
+{
     const int lb = c->nlev() - 1;
     const Geom &g = c->geom[lb];
     const int n = (int)g.n();
-    if (n > kBottomMaxDense) throw HipError{hipErrorInvalidValue, "coarsest grid too large for a dense solve"};
+    if (!c->mg_ok || c->opts.hierarchy != MPS_HIER_ALIGNED || n <= kInvRegsN) return;
     const long long ng = g.ng();
     std::vector<std::vector<double>> st(ST_N, std::vector<double>(ng, 0.0));
-    auto &B = c->L64[lb];
-    if (level_op(c, c->L64, lb) == OP_STENCIL) {
-        for (int q = 0; q < ST_N; ++q)
-            HIPCHK(hipMemcpyAsync(st[q].data(), B.st[q], ng * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    } else {
-        double *tmp[ST_N];
-        for (int q = 0; q < ST_N; ++q) {
-            tmp[q] = dalloc<double>(ng);
-            fill<double>(c, tmp[q], ng, 0.0);
-        }
-        Lev<double> v = view(c, c->L64, lb);
-        with_op(level_op(c, lb), c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
-            hipLaunchKernelGGL((k_build_stencil<double, decltype(O)::value, decltype(V)::value, decltype(R)::value>),
-                               cells_grid(g), block(), 0, c->stream, v, tmp[0], tmp[1], tmp[2], tmp[3], tmp[4], tmp[5],
-                               tmp[6], 0);
-        });
-        for (int q = 0; q < ST_N; ++q)
-            HIPCHK(hipMemcpyAsync(st[q].data(), tmp[q], ng * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (int q = 0; q < ST_N; ++q) dfree(tmp[q]);
-    }
+    RowArrays S{};
+    bottom_rows(c, S);
+    for (int q = 0; q < ST_N; ++q)
+        HIPCHK(hipMemcpyAsync(st[q].data(), S.st[q], ng * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     const int nx = g.nx, ny = g.ny, nz = g.nz;
     std::vector<double> A((size_t)n * n, 0.0), I((size_t)n * n, 0.0);
@@ -2016,6 +2049,7 @@ int mps_destroy(mps_ctx *c)
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->ev_in) (void)hipEventDestroy(c->ev_in);
+    if (c->ev_inv) (void)hipEventDestroy(c->ev_inv);
     for (auto e : c->kt_ev) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -2087,6 +2121,7 @@ int mps_create(mps_ctx **out, const mps_grid *grid, const mps_opts *opts)
         HIPCHK(hipEventCreate(&c->ev0));
         HIPCHK(hipEventCreate(&c->ev1));
         HIPCHK(hipEventCreateWithFlags(&c->ev_in, hipEventDisableTiming));
+        HIPCHK(hipEventCreateWithFlags(&c->ev_inv, hipEventDisableTiming));
         alloc_levels<double>(c, c->L64, true);
         if (c->opts.precision == MPS_PREC_FP32_DC) alloc_levels<float>(c, c->L32, true);
         const Geom &g0 = c->geom[0];
@@ -2100,8 +2135,8 @@ int mps_create(mps_ctx **out, const mps_grid *grid, const mps_opts *opts)
         c->d_dcscale = dalloc<double>(2);
         fill<double>(c, c->d_dcscale, 2, 1.0);
         HIPCHK(hipHostMalloc((void **)&c->h_scalar, 4 * sizeof(double), hipHostMallocDefault));
-        c->d_status = dalloc<int>(1);
-        fill<int>(c, c->d_status, 1, 0);
+        c->d_status = dalloc<int>(2);   // the coarse GMRES, the coarsest inverse
+        fill<int>(c, c->d_status, 2, 0);
         if (c->mg_ok) {
             const Geom &gb = c->geom.back();
             c->bottom64 = dalloc<double>(bottom_work_elems<double>((int)gb.n(), gb.ng()));
@@ -2410,15 +2445,18 @@ int mps_set_coeffs(mps_ctx *c, const double *dcoeff, const double *velx, const d
         }
         derive_coarse(c);
         conductance_coarse_levels(c);
-        for (int l = 0; l < c->nlev(); ++l) {
-            if (level_op(c, l) == OP_STENCIL) {
-                build_stencils(c, L, false);
-                break;
-            }
-        }
+        // explicit rows coarsest level first, so that its inverse (one
+        // workgroup) and the copy of its verdict are behind the host when it
+        // waits for them
+        const bool rows = level_op(c, 0) == OP_STENCIL;
+        const int lb = c->nlev() - 1;
+        if (rows) build_stencil(c, L, lb, false);
+        launch_bottom_inverse(c);
+        for (int l = lb - 1; l >= 0 && rows; --l) build_stencil(c, L, l, false);
         if (c->opts.precision == MPS_PREC_FP32_DC) build_fp32(c);
-        build_bottom_inverse(c);
+        host_bottom_inverse(c);
         HIPCHK(hipGetLastError());
+        finish_bottom_inverse(c);
         // host arrays were staged: complete before the call returns; device
         // arrays: the set-up stays ordered on the context's stream
         bool host_in = false;
@@ -3293,7 +3331,7 @@ void ensure_transpose(mps_ctx *c)
         c->LT[0].u = nullptr;
         c->LT[0].own_u = false;
     }
-    build_stencils(c, c->LT, true);
+    for (int l = 0; l < c->nlev(); ++l) build_stencil(c, c->LT, l, true);
     c->LT.back().inv = c->opts.hierarchy == MPS_HIER_ALIGNED ? c->dinvT : nullptr;
     HIPCHK(hipStreamSynchronize(c->stream));
     c->transpose_ready = true;

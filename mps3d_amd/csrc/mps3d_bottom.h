@@ -784,16 +784,21 @@ __device__ __forceinline__ void sg_weights(double cL, double cR, double DL, doub
 // the flux F = wL u_L + wR u_R (positive along +axis); row L gains F/w_L,
 // row R loses F/w_R. Physical faces keep the reference's boundary rows
 // (DIRC diffusion to the wall plus upwind outflow, ZGRD outflow). Reaction
-// and 1/dt sit on the diagonal. transpose != 0 stores A^T.
+// and 1/dt sit on the diagonal. transpose != 0 stores A^T. The FP32 cycle's
+// copy of the rows (st32, nullable) is written in the same pass. Only
+// interior entries are written: the arrays are zero from their allocation on.
+struct RowArrays {
+    double *st[ST_N];
+    float *st32[ST_N];
+};
+
 template <int OP>
-__global__ void __launch_bounds__(kBlock) k_sg_stencil(Lev<double> L, double *st0, double *st1, double *st2,
-                                                      double *st3, double *st4, double *st5, double *st6,
-                                                      int transpose)
+__global__ void __launch_bounds__(kBlock) k_sg_stencil(Lev<double> L, RowArrays S, int transpose)
 {
     int i, j, k;
     long long c;
     if (!cell_of(L, i, j, k, c)) return;
-    double *st[ST_N] = {st0, st1, st2, st3, st4, st5, st6};
+    double *const *st = S.st;
     double a[ST_N];
     for (int q = 0; q < ST_N; ++q) a[q] = 0.0;
     double d = 0.0;
@@ -832,7 +837,11 @@ __global__ void __launch_bounds__(kBlock) k_sg_stencil(Lev<double> L, double *st
     if (L.timederiv) d = d + 1.0 / L.dt;
     a[ST_C] = d;
     if (!transpose) {
-        for (int q = 0; q < ST_N; ++q) st[q][c] = a[q];
+#pragma unroll
+        for (int q = 0; q < ST_N; ++q) {
+            st[q][c] = a[q];
+            if (S.st32[q]) S.st32[q][c] = (float)a[q];
+        }
         return;
     }
     st[ST_C][c] = a[ST_C];
@@ -844,52 +853,167 @@ __global__ void __launch_bounds__(kBlock) k_sg_stencil(Lev<double> L, double *st
     if (k < L.nz) st[ST_ZM][c + L.sz] = a[ST_ZP];
 }
 
-// transposes an explicit stencil (st -> stT); stT must be zero-filled
-template <typename T>
-__global__ void __launch_bounds__(kBlock) k_transpose_stencil(Lev<T> L, const T *s0, const T *s1, const T *s2,
-                                                             const T *s3, const T *s4, const T *s5, const T *s6,
-                                                             T *t0, T *t1, T *t2, T *t3, T *t4, T *t5, T *t6)
-{
-    int i, j, k;
-    long long c;
-    if (!cell_of(L, i, j, k, c)) return;
-    t0[c] = s0[c];
-    if (i > 1) t2[c - 1] = s1[c];
-    if (i < L.nx) t1[c + 1] = s2[c];
-    if (j > 1) t4[c - L.sy] = s3[c];
-    if (j < L.ny) t3[c + L.sy] = s4[c];
-    if (k > 1) t6[c - L.sz] = s5[c];
-    if (k < L.nz) t5[c + L.sz] = s6[c];
-}
-
 // ------------------------------------------------------------------------
-// Dense inverse of the coarsest operator on the device, for the reference
-// hierarchy in fast arithmetic: the reference's coarse GMRES (m = n, one
-// restart, tol 1e-15, mgridsteps.f90:342-355) is an exact solve of the
-// coarsest system up to rounding, which x = A^-1 b gives directly
-// (k_bottom_dense, one small matrix-vector product per V-cycle).
+// Dense inverse of the coarsest operator on the device: the coarse solve of
+// a V-cycle is then one small matrix-vector product (k_bottom_dense). On
+// the reference hierarchy in fast arithmetic it stands for the reference's
+// coarse GMRES (m = n, one restart, tol 1e-15, mgridsteps.f90:342-355), which
+// is an exact solve up to rounding.
 //
-// One workgroup assembles A (row-major, n x n) from the level's 7-point rows
-// (k_build_stencil output) and inverts it in place by Gauss-Jordan
-// elimination with partial pivoting (rows swapped during the sweep, the
-// swaps undone as column swaps at the end); the matrix sits in LDS for
-// n <= kDenseLdsN, else in the global work array. Ties in the pivot search
-// go to the lowest row, so the result is deterministic. A zero pivot sets
-// *status = -1 (the inverse is then meaningless).
+// One workgroup assembles A from the level's 7-point rows and inverts it in
+// place by Gauss-Jordan elimination with partial pivoting. For n <= kInvRegsN
+// the whole matrix lives in the workgroup's registers (512 KB per CU; its
+// LDS would hold 141 rows): lane (tr, tc) of a 16 x 32 grid owns the entries
+// (tr + 16 a, tc + 32 b), a < 2 E, b < E, and a pivot step passes one column
+// and one row through LDS (two buffers, two barriers). Every wave finds the
+// pivot by itself, a maximum over keys (|value| with its low 8 bits replaced
+// by 255 - row, so near-ties go to the lowest row) in cross-lane moves of
+// the vector unit. Rows stay where they are; which row took step kk is
+// recorded and undone in the final scatter, which moves the same values as
+// swapping rows and swapping columns back. A pivot of zero (or NaN rows)
+// sets *status = -1 (the inverse is then meaningless).
+// 27 cells 21 us, 64 cells 52 us (98 us with the matrix in LDS, one column
+// per lane), 128 cells 162 us, 210 cells 480 us (2.3 us per pivot; 1024 lanes
+// with 49 entries each spill: 1000 us). On the host, with the rows copied
+// there and the inverse back, the 210-cell one held a 6.6 ms species step up
+// for more than 2 ms.
 // ------------------------------------------------------------------------
-constexpr int kDenseLdsN = 64;
+constexpr int kInvRegsN = 224;
+constexpr int kInvThreads = 512;
 constexpr int kDenseThreads = 1024;
 
-__global__ void __launch_bounds__(kDenseThreads) k_dense_inverse(Lev<double> L, const double *__restrict__ st0,
-                                                                 const double *__restrict__ st1,
-                                                                 const double *__restrict__ st2,
-                                                                 const double *__restrict__ st3,
-                                                                 const double *__restrict__ st4,
-                                                                 const double *__restrict__ st5,
-                                                                 const double *__restrict__ st6, double *gwork,
-                                                                 double *Ainv, int *status)
+// max over the wave of a key >= 0, in lane 63 (row shifts within 16 lanes,
+// then row broadcasts; lanes without a source take 0)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_max(unsigned long long v)
 {
-    __shared__ double sM[kDenseLdsN * kDenseLdsN];
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, false);
+    const unsigned long long o = ((unsigned long long)hi << 32) | lo;
+    return o > v ? o : v;
+}
+
+template <int E>
+__global__ void __launch_bounds__(kInvThreads) k_dense_inverse_regs(Lev<double> L, RowArrays S, double *Ainv,
+                                                                    double *AinvT, int *status)
+{
+    constexpr int N = 32 * E, A = 2 * E, B = E;
+    __shared__ double scol[2][N], srow[2][N];
+    __shared__ int perm[N], pos[N];
+    const int nx = L.nx, ny = L.ny, n = L.nx * L.ny * L.nz;
+    const int tid = threadIdx.x, tr = tid >> 5, tc = tid & 31, lane = tid & 63;
+    double m[A][B];
+#pragma unroll
+    for (int a = 0; a < A; ++a) {
+        const int r = tr + 16 * a;
+        const int i = r % nx + 1, j = (r / nx) % ny + 1, k = r / (nx * ny) + 1;
+        const long long c = (long long)i + (long long)L.sy * j + L.sz * k;
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int q = tc + 32 * b;
+            double v = 0.0;
+            if (r < n && q < n) {
+                if (q == r) v = S.st[ST_C][c];
+                if (i > 1 && q == r - 1) v = S.st[ST_XM][c];
+                if (i < nx && q == r + 1) v = S.st[ST_XP][c];
+                if (j > 1 && q == r - nx) v = S.st[ST_YM][c];
+                if (j < ny && q == r + nx) v = S.st[ST_YP][c];
+                if (k > 1 && q == r - nx * ny) v = S.st[ST_ZM][c];
+                if (k < L.nz && q == r + nx * ny) v = S.st[ST_ZP][c];
+            }
+            m[a][b] = v;
+        }
+    }
+    unsigned used = 0;   // bit t: row lane + 64 t has been a pivot row
+    bool bad = false;
+#pragma unroll
+    for (int KB = 0; KB < B; ++KB) {
+        for (int kc = 0; kc < 32; ++kc) {
+            const int kk = 32 * KB + kc, buf = kc & 1;
+            if (kk >= n) break;
+            if (tc == kc) {
+#pragma unroll
+                for (int a = 0; a < A; ++a) {
+                    scol[buf][tr + 16 * a] = m[a][KB];
+                    m[a][KB] = 0.0;
+                }
+            }
+            __syncthreads();
+            unsigned long long key = 0;
+#pragma unroll
+            for (int t = 0; t < (N + 63) / 64; ++t) {
+                const int r = lane + 64 * t;
+                if (r < n && !((used >> t) & 1)) {
+                    const double v = fabs(scol[buf][r]);
+                    const unsigned long long bits = v == v ? __builtin_bit_cast(unsigned long long, v) : 0;
+                    const unsigned long long w = (bits & ~0xffull) | (unsigned)(255 - r);
+                    key = w > key ? w : key;
+                }
+            }
+            key = dpp_max<0x111, 0xf>(key);   // row_shr 1, 2, 4, 8
+            key = dpp_max<0x112, 0xf>(key);
+            key = dpp_max<0x114, 0xf>(key);
+            key = dpp_max<0x118, 0xf>(key);
+            key = dpp_max<0x142, 0xa>(key);   // row_bcast 15, 31
+            key = dpp_max<0x143, 0xc>(key);
+            const unsigned klo = __builtin_amdgcn_readlane((int)key, 63);
+            const unsigned khi = __builtin_amdgcn_readlane((int)(key >> 32), 63);
+            // (an unused row below n always exists, so p < n)
+            const int p = 255 - (int)(klo & 0xffu);
+            if (khi == 0 && (klo >> 8) == 0) bad = true;
+            if ((p & 63) == lane) used |= 1u << (p >> 6);
+            const double piv = scol[buf][p];
+            const int pr = p & 15, pa = p >> 4;
+            if (tr == pr) {
+#pragma unroll
+                for (int a = 0; a < A; ++a) {
+                    if (a == pa) {
+#pragma unroll
+                        for (int b = 0; b < B; ++b) {
+                            srow[buf][tc + 32 * b] = m[a][b];
+                            m[a][b] = 0.0;
+                        }
+                    }
+                }
+            }
+            if (tid == 0) {
+                perm[kk] = p;
+                pos[p] = kk;
+            }
+            __syncthreads();
+            // the pivot row becomes rk (0 - (-1) rk), every other row loses
+            // its column entry times rk; column kk itself was set to zero
+            const double inv = 1.0 / piv;
+            double rk[B];
+#pragma unroll
+            for (int b = 0; b < B; ++b) rk[b] = ((b == KB && tc == kc) ? 1.0 : srow[buf][tc + 32 * b]) * inv;
+#pragma unroll
+            for (int a = 0; a < A; ++a) {
+                const double f = (tr == pr && a == pa) ? -1.0 : scol[buf][tr + 16 * a];
+#pragma unroll
+                for (int b = 0; b < B; ++b) m[a][b] = m[a][b] - f * rk[b];
+            }
+        }
+    }
+    // row r holds the inverse's row pos[r]; column c belongs to row perm[c] of A
+#pragma unroll
+    for (int a = 0; a < A; ++a) {
+        const int r = tr + 16 * a;
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int q = tc + 32 * b;
+            if (r < n && q < n) {
+                Ainv[(long long)pos[r] * n + perm[q]] = m[a][b];
+                if (AinvT) AinvT[(long long)perm[q] * n + pos[r]] = m[a][b];
+            }
+        }
+    }
+    if (tid == 0 && status) *status = bad ? -1 : 0;
+}
+
+// the same inverse with the matrix in global memory, for kInvRegsN < n
+__global__ void __launch_bounds__(kDenseThreads) k_dense_inverse(Lev<double> L, RowArrays S, double *gwork, double *Ainv)
+{
     __shared__ double col[kBottomMaxDense];
     __shared__ int perm[kBottomMaxDense];
     __shared__ double rv[kDenseThreads / 64];
@@ -898,99 +1022,22 @@ __global__ void __launch_bounds__(kDenseThreads) k_dense_inverse(Lev<double> L, 
     const int nx = L.nx, ny = L.ny, n = L.nx * L.ny * L.nz;
     const int tid = threadIdx.x, nt = blockDim.x;
     const long long nn = (long long)n * n;
-    // A into the matrix: called with the LDS array or the global work array
-    // itself, so each call addresses one memory kind
-    auto assemble = [&](double *M) {
-        for (long long q = tid; q < nn; q += nt) M[q] = 0.0;
-        __syncthreads();
-        for (int r = tid; r < n; r += nt) {
-            const int i = r % nx + 1, j = (r / nx) % ny + 1, k = r / (nx * ny) + 1;
-            const long long c = (long long)i + (long long)L.sy * j + L.sz * k;
-            double *row = M + (long long)r * n;
-            row[r] = st0[c];
-            if (i > 1) row[r - 1] = st1[c];
-            if (i < nx) row[r + 1] = st2[c];
-            if (j > 1) row[r - nx] = st3[c];
-            if (j < ny) row[r + nx] = st4[c];
-            if (k > 1) row[r - nx * ny] = st5[c];
-            if (k < L.nz) row[r + nx * ny] = st6[c];
-        }
-        if (tid == 0 && status) *status = 0;
-        __syncthreads();
-    };
-    if (n <= kDenseLdsN) {
-        assemble(sM);
-        // LDS-resident matrix, one column per lane. Wave 0 alone finds the
-        // pivot (a butterfly over the candidate rows, one per lane), swaps
-        // the rows and scales the pivot row, with no barrier between those
-        // steps; then every wave updates its rows (wave w of nw: rows
-        // w + nw m), each lane loading a batch of rows before it stores them
-        // (any whole number of waves: the host picks it). Two barriers
-        // per pivot. The row swaps are recorded as the original row index
-        // at each position (pos, one per lane of wave 0) and undone at the
-        // end by scattering each row's columns to their original places,
-        // which moves the same values as swapping the columns back, last
-        // swap first.
-        const int lane = tid & 63, wv = tid >> 6, nw = nt >> 6;
-        constexpr int kRows = 4;   // rows per wave and batch: all loads of a batch before its stores
-        int pos = lane;
-        for (int kk = 0; kk < n; ++kk) {
-            if (wv == 0) {
-                const int r = kk + lane;
-                double v = r < n ? fabs(sM[r * n + kk]) : -1.0;
-                if (!(v >= 0.0)) v = -1.0;   // NaN never wins
-                int bi = r;
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) {
-                    const double ov = __shfl_xor(v, off, 64);
-                    const int oi = __shfl_xor(bi, off, 64);
-                    if (ov > v || (ov == v && oi < bi)) v = ov, bi = oi;
-                }
-                const int p = bi;   // the same in every lane
-                if (lane == 0 && !(v > 0.0) && status) *status = -1;
-                const int pk = __shfl(pos, kk, 64), pp = __shfl(pos, p, 64);
-                if (lane == kk)
-                    pos = pp;
-                else if (lane == p)
-                    pos = pk;
-                double a = 0.0;
-                if (lane < n) {
-                    a = sM[kk * n + lane];
-                    if (p != kk) {
-                        const double b = sM[p * n + lane];
-                        sM[p * n + lane] = a;
-                        a = b;
-                    }
-                }
-                const double inv = 1.0 / __shfl(a, kk, 64);
-                if (lane < n) sM[kk * n + lane] = (lane == kk ? 1.0 : a) * inv;
-            }
-            __syncthreads();
-            const double rkc = lane < n ? sM[kk * n + lane] : 0.0;
-            for (int r0 = wv; r0 < n; r0 += kRows * nw) {
-                double f[kRows], x[kRows];
-#pragma unroll
-                for (int m = 0; m < kRows; ++m) {
-                    const int r = r0 + m * nw;
-                    f[m] = r < n ? sM[r * n + kk] : 0.0;
-                    x[m] = (r < n && lane < n) ? sM[r * n + lane] : 0.0;
-                }
-#pragma unroll
-                for (int m = 0; m < kRows; ++m) {
-                    const int r = r0 + m * nw;
-                    if (r < n && r != kk && lane < n) sM[r * n + lane] = (lane == kk ? 0.0 : x[m]) - f[m] * rkc;
-                }
-            }
-            __syncthreads();
-        }
-        if (wv == 0 && lane < n) perm[lane] = pos;
-        __syncthreads();
-        for (int r = wv; r < n; r += nw)
-            if (lane < n) Ainv[r * n + perm[lane]] = sM[r * n + lane];
-        return;
-    }
     double *const M = gwork;
-    assemble(M);
+    for (long long q = tid; q < nn; q += nt) M[q] = 0.0;
+    __syncthreads();
+    for (int r = tid; r < n; r += nt) {
+        const int i = r % nx + 1, j = (r / nx) % ny + 1, k = r / (nx * ny) + 1;
+        const long long c = (long long)i + (long long)L.sy * j + L.sz * k;
+        double *row = M + (long long)r * n;
+        row[r] = S.st[ST_C][c];
+        if (i > 1) row[r - 1] = S.st[ST_XM][c];
+        if (i < nx) row[r + 1] = S.st[ST_XP][c];
+        if (j > 1) row[r - nx] = S.st[ST_YM][c];
+        if (j < ny) row[r + nx] = S.st[ST_YP][c];
+        if (k > 1) row[r - nx * ny] = S.st[ST_ZM][c];
+        if (k < L.nz) row[r + nx * ny] = S.st[ST_ZP][c];
+    }
+    __syncthreads();
     for (int kk = 0; kk < n; ++kk) {
         // pivot: the largest |M[r][kk]|, r >= kk, lowest r on ties
         double best = -1.0;
@@ -1013,7 +1060,6 @@ __global__ void __launch_bounds__(kDenseThreads) k_dense_inverse(Lev<double> L, 
                 if (rv[w] > b || (rv[w] == b && ri[w] < p)) b = rv[w], p = ri[w];
             piv = p;
             perm[kk] = p;
-            if (!(b > 0.0) && status) *status = -1;
         }
         __syncthreads();
         const int p = piv;

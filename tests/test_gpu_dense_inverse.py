@@ -1,0 +1,59 @@
+"""The coarsest level's dense inverse (k_dense_inverse_regs, and the paths for
+larger grids) on grids that are their own coarsest level: the solve is then
+x = A^-1 b, compared with numpy's dense solve of the matrix that find_AX
+gives. Bar: 8 n eps cond(A) relative, the forward error of an inverse formed
+by elimination with partial pivoting and applied by one product, with a
+factor for its constants. Sizes: one cell, the edges of each register
+layout, and above the largest."""
+import numpy as np
+import pytest
+
+from mps3d_amd import FieldSolver, _lib as M, ghosted
+from mps3d_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1, 1), (3, 3, 3), (4, 4, 2), (3, 11, 1), (4, 4, 4), (5, 13, 1), (8, 4, 4), (3, 43, 1), (7, 5, 6), (8, 7, 4),
+         (15, 15, 1)]
+
+
+def dense(s, n):
+    N = int(np.prod(n))
+    A = np.empty((N, N))
+    for q in range(N):
+        e = np.zeros(N)
+        e[q] = 1.0
+        A[:, q] = s.find_AX(ghosted(e.reshape(n, order="F")))[0].ravel(order="F")
+    return A
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("form", ["aligned_sg", "aligned_cdr", "aligned_diffusion", "ref_fast"])
+def test_coarsest_solve_is_the_dense_solve(gpu, n, form):
+    c = W.random_cdr(n, seed=17 + sum(n))
+    if form == "aligned_diffusion":
+        c.velx = c.vely = c.velz = None
+    # a reaction of either sign as large as the diffusive rows: the diagonal
+    # does not dominate, so rows are exchanged
+    c.reac = 400.0 * c.reac
+    kw = {"ref_fast": dict(hierarchy="ref", p=n, arith="fast"),
+          "aligned_sg": dict(hierarchy="aligned", flux="sg", arith="fast")}.get(form, dict(hierarchy="aligned", arith="fast"))
+    if form == "ref_fast":
+        c.velx = c.vely = c.velz = None
+    b = np.random.default_rng(2).standard_normal(n)
+    with FieldSolver(c.n, c.length, tol=1e-8, tol_kind="rel", max_cycles=1, **kw) as s:
+        s.set_case(c)
+        A = dense(s, n)
+        x = ghosted(np.zeros(n))
+        s.solve_rhs(b, x)
+    ref = np.linalg.solve(A, b.ravel(order="F"))
+    err = np.linalg.norm(x[1:-1, 1:-1, 1:-1].ravel(order="F") - ref) / np.linalg.norm(ref)
+    assert err <= 8 * b.size * np.finfo(float).eps * np.linalg.cond(A)
+
+
+@pytest.mark.parametrize("n", [(3, 3, 3), (8, 7, 4), (15, 15, 1)])
+def test_a_singular_coarsest_operator_is_refused(gpu, n):
+    with FieldSolver(n, hierarchy="aligned", arith="fast") as s:
+        s.set_bc(("ZGRD",) * 6)
+        with pytest.raises(M.MpsError, match="singular"):
+            s.set_coeffs(np.zeros(n))
