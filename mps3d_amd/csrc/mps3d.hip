@@ -9,6 +9,7 @@
 #include "mps3d_sweep.h"
 #include "mps3d_sweep2.h"
 #include "mps3d_lds_cycle.h"
+#include "mps3d_tail.h"
 #include "mps3d_transport.h"
 #include "mps3d_stream.h"
 
@@ -130,6 +131,7 @@ struct LevelBuf {
     double *w[3] = {};
     T *u2 = nullptr;              // ping-pong partner of u for fused sweeps
     const double *inv = nullptr;  // dense inverse of the coarsest operator
+    T *rows = nullptr;            // formed rows of a small level (k_tail_rows)
     bool own_u = true;
     int op = -1;  // operator form override (>= 0), e.g. transposed stencils
 };
@@ -197,6 +199,7 @@ struct mps_ctx {
     hipEvent_t ev_in = nullptr;          // orders calls after the null stream
     hipEvent_t ev_inv = nullptr;         // the coarsest inverse's status has been copied
     bool inv_pending = false;            // and set_coeffs has yet to read it
+    bool tail_dirty = true;              // coefficients or BC codes changed since k_tail_rows
     double last_ms = 0.0;
     int last_cycles = 0;
     double *dinv = nullptr;              // dense inverse of the coarsest operator
@@ -534,6 +537,7 @@ void free_levels(std::vector<LevelBuf<T>> &L)
         for (int q = 1; q < 4; ++q) dfree(B.fc[q]);
         for (auto p : B.faces) dfree(p);
         for (auto p : B.w) dfree(p);
+        dfree(B.rows);
     }
     L.clear();
 }
@@ -1157,6 +1161,96 @@ void launch_lds_cycle(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l)
     hipLaunchKernelGGL(k_lds_cycle<T>, dim3(1), dim3(kLdsBlock), (size_t)(words * sizeof(T)), c->stream, S);
 }
 
+// ------------------------------------ small levels of the reference hierarchy
+// k_tail_down and k_tail_up take the reference hierarchy's V-cycle over from
+// the first level of at most kTailCells cells above the coarsest (-1: none):
+// what a level of that size costs is launches and latency, and its state no
+// longer fits one workgroup's registers and LDS above it.
+int tail_from(const mps_ctx *c)
+{
+    if (c->opts.hierarchy != MPS_HIER_REF) return -1;
+    const int lb = c->nlev() - 1;
+    // (every level below the first is held with its ghosts as well)
+    int l = lb;
+    while (l > 0 && c->geom[l - 1].n() <= kTailCells && c->geom[l].ng() <= kTailGhosted && lb - l + 2 <= kTailLev) --l;
+    return l < lb ? l : -1;
+}
+
+// forms those levels' rows if the coefficients or the boundary codes changed
+// since the last time (levels of explicit rows have them already)
+template <typename T>
+void tail_rows(mps_ctx *c, std::vector<LevelBuf<T>> &L)
+{
+    const int l = tail_from(c);
+    if (l < 0 || L.empty() || level_op(c, L, l) == OP_STENCIL) return;
+    TailLevels<T> A{};
+    A.nlev = c->nlev() - l;
+    for (int q = 0; q < A.nlev; ++q) {
+        LevelBuf<T> &B = L[l + q];
+        if (!B.rows) B.rows = dalloc<T>((size_t)c->geom[l + q].n() * kTailRowArrays);
+        A.L[q] = view(c, L, l + q);
+        A.rows[q] = B.rows;
+    }
+    auto go = [&](auto V, auto R, auto F) {
+        hipLaunchKernelGGL((k_tail_rows<T, decltype(V)::value, decltype(R)::value, decltype(F)::value>),
+                           dim3((unsigned)((c->geom[l].n() + kBlock - 1) / kBlock), (unsigned)A.nlev), block(), 0,
+                           c->stream, A);
+    };
+    const BoolC<true> yes{};
+    const BoolC<false> no{};
+    if (A.L[0].fast && c->has_reac) go(no, yes, yes);
+    else if (A.L[0].fast) go(no, no, yes);
+    else if (c->has_vel && c->has_reac) go(yes, yes, no);
+    else if (c->has_vel) go(yes, no, no);
+    else if (c->has_reac) go(no, yes, no);
+    else go(no, no, no);
+}
+void prepare_tail(mps_ctx *c)
+{
+    if (!c->tail_dirty) return;
+    tail_rows<double>(c, c->L64);
+    tail_rows<float>(c, c->L32);
+    c->tail_dirty = false;
+}
+
+// level l's part of the cycle: down to the coarsest right-hand side (up 0), or
+// back from the coarsest solution (up 1)
+template <typename T>
+void launch_tail(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, bool homog, bool up)
+{
+    TailLevels<T> A{};
+    A.nlev = c->nlev() - l;
+    A.nu = up ? c->opts.nu2 : c->opts.nu1;
+    for (int q = 0; q < A.nlev; ++q) {
+        A.L[q] = view(c, L, l + q);
+        A.u[q] = L[l + q].u;
+        A.uold[q] = L[l + q].uold;
+        A.b[q] = L[l + q].b;
+        A.rows[q] = L[l + q].rows;
+        for (int f = 0; f < 6; ++f) A.face[q][f] = homog ? nullptr : L[l + q].faces[f];
+    }
+    auto go = [&](auto O, auto V, auto R, auto F) {
+        if (up)
+            hipLaunchKernelGGL((k_tail_up<T, decltype(O)::value, decltype(V)::value, decltype(R)::value,
+                                          decltype(F)::value>),
+                               dim3(1), dim3(kTailThreads), 0, c->stream, A);
+        else
+            hipLaunchKernelGGL((k_tail_down<T, decltype(O)::value, decltype(V)::value, decltype(R)::value,
+                                            decltype(F)::value>),
+                               dim3(1), dim3(kTailThreads), 0, c->stream, A);
+    };
+    const bool fast = A.L[0].fast != 0;   // rows without convection only
+    const BoolC<true> yes{};
+    const BoolC<false> no{};
+    if (level_op(c, L, l) == OP_STENCIL) go(IntC<OP_STENCIL>{}, no, no, yes);
+    else if (fast && c->has_reac) go(IntC<OP_REF>{}, no, yes, yes);
+    else if (fast) go(IntC<OP_REF>{}, no, no, yes);
+    else if (c->has_vel && c->has_reac) go(IntC<OP_REF>{}, yes, yes, no);
+    else if (c->has_vel) go(IntC<OP_REF>{}, yes, no, no);
+    else if (c->has_reac) go(IntC<OP_REF>{}, no, yes, no);
+    else go(IntC<OP_REF>{}, no, no, no);
+}
+
 // --------------------------------------------------------------- V-cycle
 // One V-cycle from level l down (perform_vcycle, mgridsteps.f90:384-579).
 // Level l's b must hold its right-hand side.
@@ -1175,6 +1269,14 @@ void vcycle(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, T *bwork, bool homog
     }
     if (l > 0 && l == lds_cycle_from<T>(c, L)) {
         launch_lds_cycle<T>(c, L, l);
+        return;
+    }
+    if (l == tail_from(c)) {
+        if (zero_u) fill<T>(c, L[l].u, g.ng(), T(0));
+        const int lb = c->nlev() - 1;
+        launch_tail<T>(c, L, l, homog, false);
+        launch_bottom<T>(c, L, lb, level_op(c, L, lb), bwork);
+        launch_tail<T>(c, L, l, homog, true);
         return;
     }
     bool zg = false;
@@ -1751,6 +1853,7 @@ int solve_core(mps_ctx *c, double *u, double *b, bool homog, double *history, do
         explicit RelaxScope(mps_ctx *c_) : c(c_) { c->relax_now = true; }
         ~RelaxScope() { c->relax_now = false; }
     } relax(c);
+    prepare_tail(c);
     double bn2 = 0.0;
     const bool dc = c->opts.precision == MPS_PREC_FP32_DC;
     if (c->opts.tol_kind == MPS_TOL_REL_L2 || dc) {
@@ -2306,6 +2409,7 @@ void set_bc_device(mps_ctx *c, const double *const faces[6])
 int mps_set_bc(mps_ctx *c, const int codes[6], const double *const faces[6])
 {
     if (!c || !codes) return fail(MPS_ERR_ARG, "null argument");
+    c->tail_dirty = true;
     try {
         HIPCHK(hipSetDevice(c->device));
         for (int f = 0; f < 6; ++f) {
@@ -2401,6 +2505,7 @@ int mps_set_coeffs(mps_ctx *c, const double *dcoeff, const double *velx, const d
 {
     if (!c) return fail(MPS_ERR_ARG, "null context");
     if (timederiv && !(dt != 0.0)) return fail(MPS_ERR_ARG, "timederiv with dt = 0");
+    c->tail_dirty = true;
     try {
         HIPCHK(hipSetDevice(c->device));
         if (int st = after_null_stream(c)) return st;
@@ -3110,6 +3215,7 @@ int mps_vcycle(mps_ctx *c, double *soln, const double *sterm, double *resnorm)
         double *u = bind_solution(c, soln, staged);
         fill<int>(c, c->d_status, 1, 0);
         compute_b0(c, stage_interior(c, sterm));
+        prepare_tail(c);
         fp64_cycle(c, u);
         double ss = c->geom[0].bottom ? 0.0 : read_scalar(c);
         HIPCHK(hipMemcpyAsync(c->h_scalar + 1, c->d_status, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -3562,6 +3668,7 @@ int mps_gmres(mps_ctx *c, const double *b, double *x, int m, int max_restarts, d
         // ---------------- FGMRES(m), right-preconditioned by one V-cycle
         if (m + 1 > kMaxVec) return fail(MPS_ERR_ARG, "m at most %d", kMaxVec - 1);
         if (!c->mg_ok) return fail(MPS_ERR_ARG, "no multigrid hierarchy for this grid: %s", c->mg_error.c_str());
+        prepare_tail(c);
         GmresBufs &G = gmres_bufs(c, m);
         const double *bd = stage_interior(c, b);
         Lev<double> v0 = view(c, c->L64, 0);
