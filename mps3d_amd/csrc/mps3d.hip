@@ -8,7 +8,7 @@
 #include "mps3d_kernels.h"
 #include "mps3d_sweep.h"
 #include "mps3d_sweep2.h"
-#include "mps3d_lds_cycle.h"
+#include "mps3d_small.h"
 #include "mps3d_tail.h"
 #include "mps3d_transport.h"
 #include "mps3d_stream.h"
@@ -1114,51 +1114,72 @@ bool zero_first_ok(const mps_ctx *c, const std::vector<LevelBuf<T>> &L, int l, i
     return first_fused && fused_ok(c, L, l, op) && (op == OP_STENCIL || view(c, L, l).fast);
 }
 
-// ---------------------------------------------- LDS-resident small levels
-// k_lds_cycle takes over the V-cycle from the first level whose levels down
-// to the coarsest fit kLdsBudget bytes of LDS: aligned hierarchy with
-// explicit-stencil (conductance) coarse rows and a dense coarsest solve.
-constexpr long long kLdsBudget = 64 * 1024;
-
+// ------------------------------------- small levels of the aligned hierarchy
+// k_small_cycle takes the V-cycle over from the first level from which all
+// levels down to the coarsest fit its LDS (and its lanes' cells): explicit-
+// stencil rows (conductance or Scharfetter-Gummel) and a dense coarsest
+// solve of no more rows than lanes.
 template <typename T>
-int lds_cycle_from(const mps_ctx *c, const std::vector<LevelBuf<T>> &L)
+int small_cycle_from(const mps_ctx *c, const std::vector<LevelBuf<T>> &L)
+{
+    if (c->opts.hierarchy != MPS_HIER_ALIGNED || !L.back().inv) return -1;
+    const int lb = c->nlev() - 1;
+    if (c->geom[lb].n() > kSmallHalf) return -1;
+    long long bytes = 0;
+    int from = lb;
+    for (int l = lb; l >= 1 && lb - l + 1 <= kSmallLev; --l) {
+        const Geom &g = c->geom[l];
+        if (level_op(c, L, l) != OP_STENCIL || g.n() > (1 << 15)) break;
+        bytes += small_level_bytes<T>(g.nx, g.ny, g.nz);
+        if (bytes > kSmallBytes || (g.nx + 1) / 2 * g.ny * g.nz > kSmallThreads ||
+            3 * std::max(g.nx, std::max(g.ny, g.nz)) > kSmallHalf)
+            break;
+        from = l;
+    }
+    return from < lb ? from : -1;
+}
+
+// The smallest levels, whose u, b, r and seven rows each, all levels down to
+// the coarsest together, take at most 64 KB: a full-multigrid pass starts on
+// the first of them, and they sweep with plain Gauss-Seidel in every solve
+// (over-relaxation gains nothing there).
+template <typename T>
+int plain_from(const mps_ctx *c, const std::vector<LevelBuf<T>> &L)
 {
     if (c->opts.hierarchy != MPS_HIER_ALIGNED || !L.back().inv) return -1;
     long long words = 0;
     int from = -1;
     for (int l = c->nlev() - 1; l >= 1; --l) {
         if (level_op(c, L, l) != OP_STENCIL) break;
-        const Geom &g = c->geom[l];
-        words += lds_level_words(g.nx, g.ny, g.nz);
-        if (words * (long long)sizeof(T) > kLdsBudget || c->nlev() - l > kLdsMaxLev) break;
+        words += c->geom[l].ng() + (2 + ST_N) * c->geom[l].n();
+        if (words * (long long)sizeof(T) > 64 * 1024 || c->nlev() - l > 4) break;
         from = l;
     }
     return (from >= 0 && from < c->nlev() - 1) ? from : -1;
 }
 
 template <typename T>
-void launch_lds_cycle(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l)
+void launch_small_cycle(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, bool zero)
 {
-    LdsLevels<T> S{};
-    S.nlev = c->nlev() - l;
-    long long words = 0;
-    for (int q = 0; q < S.nlev; ++q) {
-        const Geom &g = c->geom[l + q];
-        S.nx[q] = g.nx, S.ny[q] = g.ny, S.nz[q] = g.nz;
-        for (int s = 0; s < ST_N; ++s) S.st[q][s] = L[l + q].st[s];
-        S.W[q] = AlignedW{L[l + q].w[0], L[l + q].w[1], L[l + q].w[2]};
-        words += lds_level_words(g.nx, g.ny, g.nz);
+    SmallLevels<T> A{};
+    A.nlev = c->nlev() - l;
+    const int plain = plain_from<T>(c, L);
+    for (int q = 0; q < A.nlev; ++q) {
+        A.L[q] = view(c, L, l + q);
+        A.W[q] = AlignedW{L[l + q].w[0], L[l + q].w[1], L[l + q].w[2]};
+        A.omega[q] = plain >= 0 && l + q >= plain ? T(1) : A.L[q].omega;
     }
-    const Geom &g0 = c->geom[l];
-    S.b0 = L[l].b;
-    S.u0 = L[l].u;
-    S.sy0 = g0.nx + 2;
-    S.sz0 = (long long)(g0.nx + 2) * (g0.ny + 2);
-    S.inv = L.back().inv;
-    S.nu1 = c->opts.nu1;
-    S.nu2 = c->opts.nu2;
-    S.fast = view(c, L, l).fast;
-    hipLaunchKernelGGL(k_lds_cycle<T>, dim3(1), dim3(kLdsBlock), (size_t)(words * sizeof(T)), c->stream, S);
+    A.u0 = L[l].u;
+    A.b0 = L[l].b;
+    A.invT = L.back().inv == c->dinv ? c->dinvT : c->dinv;
+    A.nu1 = c->opts.nu1;
+    A.nu2 = c->opts.nu2;
+    A.zero = zero ? 1 : 0;
+    const Geom &g = c->geom[l];
+    if ((g.nx + 1) / 2 * g.ny * g.nz <= kSmallHalf)
+        hipLaunchKernelGGL((k_small_cycle<T, kSmallHalf>), dim3(1), dim3(kSmallHalf), 0, c->stream, A);
+    else
+        hipLaunchKernelGGL((k_small_cycle<T, kSmallThreads>), dim3(1), dim3(kSmallThreads), 0, c->stream, A);
 }
 
 // ------------------------------------ small levels of the reference hierarchy
@@ -1267,8 +1288,8 @@ void vcycle(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, T *bwork, bool homog
         launch_bottom<T>(c, L, l, op, bwork);
         return;
     }
-    if (l > 0 && l == lds_cycle_from<T>(c, L)) {
-        launch_lds_cycle<T>(c, L, l);
+    if (const int small = small_cycle_from<T>(c, L); small >= 0 && l >= small) {
+        launch_small_cycle<T>(c, L, l, zero_u);
         return;
     }
     if (l == tail_from(c)) {
@@ -1353,7 +1374,7 @@ template <typename T>
 void fmg(mps_ctx *c, std::vector<LevelBuf<T>> &L, T *bwork)
 {
     const int nl = c->nlev();
-    int top = lds_cycle_from<T>(c, L);
+    int top = plain_from<T>(c, L);
     if (top < 0) top = nl - 1;
     for (int l = 0; l < top; ++l) launch_restrict_fw<T>(c, L, l, L[l].b);
     vcycle<T>(c, L, top, bwork, true, true);
