@@ -485,6 +485,46 @@ int mps_time_in_solve(mps_ctx *ctx, int kernel, int fp32, double *soln, int *ncy
  * reads and writes. */
 int mps_time_stream(int kind, long long bytes_per_array, int reps, double *avg_ms, double *bytes);
 
+/* Field passes of the differentiable solves and of the multi-species
+ * discharge step (no reference counterpart; the step's order is
+ * solve_manager.f90:405-477). They take device arrays and run on `stream`
+ * (a hipStream_t of the current device, NULL the default stream), without
+ * synchronising. Fields are (nx, ny, nz) interior arrays, x fastest. */
+#define MPS_PAD_FIELDS 4
+#define MPS_DIS_SPECIES 8
+#define MPS_DIS_REACTIONS 8
+#define MPS_DIS_ORDER 4
+
+/* dst: k ghosted fields one after the other, ghosts zero, the interior of
+ * field f scale * src[f]. */
+int mps_pad_fields(void *stream, int nx, int ny, int nz, int k, const double *const *src, double scale, double *dst);
+
+typedef struct {
+    int nspecies, nreactions;
+    int electron;                    /* index of the species whose outflow is at T_e (-1 none) */
+    int energy;                      /* with the electron energy equation */
+    int outflow[MPS_DIS_SPECIES];    /* thermal outflow through the z faces */
+    int arrhenius[MPS_DIS_REACTIONS];/* rate exp(-ea / mean energy), else rate */
+    int order[MPS_DIS_REACTIONS];    /* reactants */
+    int reactant[MPS_DIS_REACTIONS][MPS_DIS_ORDER]; /* species, -1 the background gas */
+    double nu[MPS_DIS_SPECIES][MPS_DIS_REACTIONS];  /* net production per event */
+    double rate[MPS_DIS_REACTIONS], ea[MPS_DIS_REACTIONS], loss[MPS_DIS_REACTIONS];
+    double charge[MPS_DIS_SPECIES], cbar[MPS_DIS_SPECIES]; /* thermal speed of the others */
+    double cbar_num, cbar_den;       /* the electrons': sqrt(cbar_num T_e / cbar_den) */
+    double rho_coef, wall_weight;    /* of the potential's right-hand side */
+    double dt, h, gas, eps0, eps_ref, T_gas, mu_e, elastic;
+    const double *dens[MPS_DIS_SPECIES];
+    const double *neps, *phi, *eps_r, *lo, *hi;
+    double *E;                       /* out: E_x, E_y, E_z */
+    double *rhs;                     /* out: each species, then the electron energy */
+} mps_discharge;
+
+/* rhs: the potential's right-hand side rho_coef * sum charge * dens plus the
+ * electrode potentials lo and hi in the first and last plane. */
+int mps_charge_rhs(void *stream, int nx, int ny, int nz, const mps_discharge *d, double *rhs);
+/* E and every right-hand side of d from phi and the old state. */
+int mps_discharge_rhs(void *stream, int nx, int ny, int nz, const mps_discharge *d);
+
 /* The context's HIP stream (hipStream_t), for callers that order work
  * against it. */
 void *mps_stream(mps_ctx *ctx);

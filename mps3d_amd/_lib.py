@@ -34,7 +34,10 @@ EXPORTS = (
     "mps_time_in_solve",
     "mps_get_grid", "mps_gmres_noalloc", "mps_restrict", "mps_prolong1",
     "mps_eden_faces", "mps_neutral_faces", "mps_eenergy_faces", "mps_floor", "mps_set_source",
+    "mps_pad_fields", "mps_charge_rhs", "mps_discharge_rhs",
 )
+# sizes of mps_pad_fields and mps_discharge
+PAD_FIELDS, DIS_SPECIES, DIS_REACTIONS, DIS_ORDER = 4, 8, 8, 4
 
 
 _dp = C.POINTER(C.c_double)
@@ -62,6 +65,22 @@ class Opts(C.Structure):
                 ("nu1", C.c_int), ("nu2", C.c_int), ("max_cycles", C.c_int),
                 ("tol", C.c_double), ("tol_kind", C.c_int), ("arith", C.c_int), ("start", C.c_int),
                 ("dc_inner", C.c_int), ("omega", C.c_double)]
+
+
+class Discharge(C.Structure):
+    """mps_discharge: one step's parameters and device fields."""
+    _fields_ = [("nspecies", C.c_int), ("nreactions", C.c_int), ("electron", C.c_int), ("energy", C.c_int),
+                ("outflow", C.c_int * DIS_SPECIES), ("arrhenius", C.c_int * DIS_REACTIONS),
+                ("order", C.c_int * DIS_REACTIONS), ("reactant", (C.c_int * DIS_ORDER) * DIS_REACTIONS),
+                ("nu", (C.c_double * DIS_REACTIONS) * DIS_SPECIES), ("rate", C.c_double * DIS_REACTIONS),
+                ("ea", C.c_double * DIS_REACTIONS), ("loss", C.c_double * DIS_REACTIONS),
+                ("charge", C.c_double * DIS_SPECIES), ("cbar", C.c_double * DIS_SPECIES),
+                ("cbar_num", C.c_double), ("cbar_den", C.c_double),
+                ("rho_coef", C.c_double), ("wall_weight", C.c_double), ("dt", C.c_double), ("h", C.c_double),
+                ("gas", C.c_double), ("eps0", C.c_double), ("eps_ref", C.c_double), ("T_gas", C.c_double),
+                ("mu_e", C.c_double), ("elastic", C.c_double),
+                ("dens", _vp * DIS_SPECIES), ("neps", _vp), ("phi", _vp), ("eps_r", _vp), ("lo", _vp), ("hi", _vp),
+                ("E", _vp), ("rhs", _vp)]
 
 
 _lib = None
@@ -118,6 +137,9 @@ def load():
     L.mps_eenergy_faces.argtypes = [_vp, C.POINTER(C.c_int), _vp, _vp, C.c_double, _vp, C.c_double, _vp]
     L.mps_floor.argtypes = [_vp, _vp, C.c_double]
     L.mps_set_source.argtypes = [_vp, _vp]
+    L.mps_pad_fields.argtypes = [_vp] + [C.c_int] * 4 + [C.POINTER(_vp), C.c_double, _vp]
+    L.mps_charge_rhs.argtypes = [_vp] + [C.c_int] * 3 + [C.POINTER(Discharge), _vp]
+    L.mps_discharge_rhs.argtypes = [_vp] + [C.c_int] * 3 + [C.POINTER(Discharge)]
     L.mps_restrict.argtypes = [_vp, _vp, _vp]
     L.mps_prolong1.argtypes = [_vp, _vp, _vp]
     L.mps_get_grid.argtypes = [_vp, C.POINTER(Grid), C.POINTER(C.c_int)]

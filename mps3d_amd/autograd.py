@@ -20,6 +20,7 @@ from __future__ import annotations
 import ctypes as C
 
 import torch
+from torch.autograd import forward_ad as fwAD
 
 from . import _lib as M
 from .solver import FieldSolver
@@ -32,6 +33,36 @@ def pad(t):
 
 def interior(g):
     return g[1:-1, 1:-1, 1:-1]
+
+
+def native_fields(shape, *fields):
+    """Whether the library's field passes can take these tensors by address:
+    contiguous float64 fields of that shape on the current GPU, outside
+    tracing, functorch transforms, forward-mode levels and dispatch modes
+    (which see tensor operations only)."""
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active():
+        return False
+    if fwAD._current_level >= 0 or torch._C._len_torch_dispatch_stack() or max(shape) > 16000:
+        return False
+    dev = torch.cuda.current_device()
+    return all(type(t) is torch.Tensor and t.is_cuda and t.device.index == dev and t.dtype == torch.float64 and
+               tuple(t.shape) == tuple(shape) and t.is_contiguous() and not t.is_neg() for t in fields)
+
+
+def pad_fields(fields, scale=1.0):
+    """scale * each interior field, zero-ghosted, as one (k, nz+2, ny+2, nx+2)
+    tensor made in one pass, or as a list of padded tensors where the fields
+    are not the library's to read."""
+    fields = [t.detach() for t in fields]
+    shape = tuple(fields[0].shape) if fields else ()
+    if len(shape) != 3 or not 0 < len(fields) <= M.PAD_FIELDS or not fields[0].is_cuda or not native_fields(shape, *fields):
+        return [pad(t if scale == 1.0 else scale * t) for t in fields]
+    nz, ny, nx = shape
+    out = torch.empty((len(fields), nz + 2, ny + 2, nx + 2), dtype=torch.float64, device=fields[0].device)
+    src = (C.c_void_p * len(fields))(*[t.data_ptr() for t in fields])
+    M.check(M.load().mps_pad_fields(torch.cuda.current_stream().cuda_stream, nx, ny, nz, len(fields), src, scale,
+                                    out.data_ptr()))
+    return out
 
 
 class Operator:
@@ -73,9 +104,9 @@ class Operator:
         self._rhs = None
         self.cycles = []
 
-    def configure(self, vel=None, rhs=None):
-        """Sets the operator for velocities vel (3 interior tensors or None)
-        and the right-hand side rhs (interior, or None for zero). Without
+    def configure(self, vel=None, rhs=None, scale=1.0):
+        """Sets the operator for velocities scale * vel (3 interior tensors or
+        None) and the right-hand side rhs (interior, or None for zero). Without
         velocities the operator is the same every time, so its coefficients
         (and the hierarchy built from them) are set once; the right-hand
         side goes to the solve itself."""
@@ -84,13 +115,14 @@ class Operator:
                 self.solver.set_coeffs(self.D, None, None, None, self.reac, self._zero, self.timederiv, self.dt)
                 self._static = True
         else:
-            vg = tuple(pad(v.detach()) if v is not None else self._zero for v in vel)
+            placed = iter(pad_fields([v for v in vel if v is not None], scale))
+            vg = tuple(next(placed) if v is not None else self._zero for v in vel)
             self.solver.set_coeffs(self.D, *vg, self.reac, self._zero, self.timederiv, self.dt)
             self._static = False
         self._rhs = None if rhs is None else rhs.detach().contiguous()
 
     def solve(self, x0=None):
-        x = torch.zeros_like(self.D) if x0 is None else pad(x0.detach())
+        x = torch.zeros_like(self.D) if x0 is None else pad_fields([x0])[0]
         b = self._rhs if self._rhs is not None else torch.zeros(self.n[::-1], dtype=torch.float64, device=x.device)
         if self.method == "gmres":
             k, r, st = self.solver.gmres(b, x, m=self.gmres_m, restarts=self.gmres_restarts, tol=self.tol)
@@ -101,6 +133,11 @@ class Operator:
                 r, k, "iterations" if self.method == "gmres" else "cycles"))
         self.cycles.append(k)
         return x
+
+    def advance(self, rhs, x0, vel=None, scale=1.0):
+        """The interior solution for velocities scale * vel, outside autograd."""
+        self.configure(vel, rhs, scale)
+        return interior(self.solve(x0)).clone()
 
     def solve_transpose(self, g):
         lam = torch.zeros_like(self.D)

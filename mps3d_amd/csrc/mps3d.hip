@@ -5,6 +5,7 @@
 // stream and reads back one residual norm per cycle.
 #include "../../include/mps3d.h"
 #include "mps3d_bottom.h"
+#include "mps3d_discharge.h"
 #include "mps3d_kernels.h"
 #include "mps3d_sweep.h"
 #include "mps3d_sweep2.h"
@@ -4222,4 +4223,63 @@ extern "C" int mps_grad_velocity(mps_ctx *c, const double *lam, const double *x,
         return fail(MPS_ERR_HIP, "%s: %s", e.what, hipGetErrorString(e.e));
     }
     return MPS_OK;
+}
+
+// ------------------------------------------------------------ field passes
+extern "C" int mps_pad_fields(void *stream, int nx, int ny, int nz, int k, const double *const *src, double scale,
+                              double *dst)
+{
+    if (nx < 1 || ny < 1 || nz < 1 || k < 1 || k > MPS_PAD_FIELDS || !src || !dst ||
+        (long long)k * (nz + 2) > 65535 || (ny + 1) / kDisY + 1 > 65535)
+        return fail(MPS_ERR_ARG, "bad arguments");
+    PadSet P{};
+    for (int f = 0; f < k; ++f) {
+        if (!src[f]) return fail(MPS_ERR_ARG, "null field");
+        P.src[f] = src[f];
+    }
+    P.dst = dst;
+    hipLaunchKernelGGL(k_pad_fields, dim3((nx + 1) / kDisX + 1, (ny + 1) / kDisY + 1, k * (nz + 2)),
+                       dim3(kDisX, kDisY), 0, (hipStream_t)stream, P, nx, ny, nz, scale);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? MPS_OK : fail(MPS_ERR_HIP, "%s", hipGetErrorString(e));
+}
+
+namespace {
+
+int discharge_bad(int nx, int ny, int nz, const mps_discharge *d)
+{
+    if (nx < 1 || ny < 1 || nz < 2 || nz > 65535 || (ny - 1) / kDisY + 1 > 65535 || !d) return 1;
+    if (d->nspecies < 1 || d->nspecies > MPS_DIS_SPECIES || d->nreactions < 0 || d->nreactions > MPS_DIS_REACTIONS)
+        return 1;
+    if (d->electron >= d->nspecies || (d->energy && (d->electron < 0 || !d->neps)) || !d->lo || !d->hi) return 1;
+    for (int s = 0; s < d->nspecies; ++s)
+        if (!d->dens[s]) return 1;
+    for (int r = 0; r < d->nreactions; ++r) {
+        if (d->order[r] < 0 || d->order[r] > MPS_DIS_ORDER) return 1;
+        for (int m = 0; m < d->order[r]; ++m)
+            if (d->reactant[r][m] < -1 || d->reactant[r][m] >= d->nspecies) return 1;
+    }
+    return 0;
+}
+
+dim3 discharge_grid(int nx, int ny, int nz) { return dim3((nx - 1) / kDisX + 1, (ny - 1) / kDisY + 1, nz); }
+
+}  // namespace
+
+extern "C" int mps_charge_rhs(void *stream, int nx, int ny, int nz, const mps_discharge *d, double *rhs)
+{
+    if (discharge_bad(nx, ny, nz, d) || !d->eps_r || !rhs) return fail(MPS_ERR_ARG, "bad arguments");
+    hipLaunchKernelGGL(k_charge_rhs, discharge_grid(nx, ny, nz), dim3(kDisX, kDisY), 0, (hipStream_t)stream, *d, rhs,
+                       nx, ny, nz);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? MPS_OK : fail(MPS_ERR_HIP, "%s", hipGetErrorString(e));
+}
+
+extern "C" int mps_discharge_rhs(void *stream, int nx, int ny, int nz, const mps_discharge *d)
+{
+    if (discharge_bad(nx, ny, nz, d) || !d->phi || !d->E || !d->rhs) return fail(MPS_ERR_ARG, "bad arguments");
+    hipLaunchKernelGGL(k_discharge_rhs, discharge_grid(nx, ny, nz), dim3(kDisX, kDisY), 0, (hipStream_t)stream, *d,
+                       nx, ny, nz);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? MPS_OK : fail(MPS_ERR_HIP, "%s", hipGetErrorString(e));
 }

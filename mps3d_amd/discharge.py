@@ -28,9 +28,10 @@ One step, in the order of plasma_pde/solve_manager.f90:405-477:
 Species solves are FGMRES(30) preconditioned by one V-cycle (``method=
 "gmres"``), Poisson iterates V-cycles; with ``precision="fp32dc"`` both
 smooth in FP32 under FP64 residuals. Boundary data enter through the
-right-hand sides, which torch builds, so torch autograd differentiates the
-whole run, every linear solve by the hand-written adjoint
-(:class:`mps3d_amd.autograd.LinearSolve`). Fields are float64 (nz, ny, nx)
+right-hand sides. Where a gradient is wanted torch builds these, so torch
+autograd differentiates the whole run, every linear solve by the hand-written
+adjoint (:class:`mps3d_amd.autograd.LinearSolve`); else the library's field
+passes do, with the same arithmetic in the same order. Fields are float64 (nz, ny, nx)
 tensors on the GPU; units are SI with energies and temperatures in eV.
 """
 from __future__ import annotations
@@ -43,7 +44,8 @@ import numpy as np
 import torch
 from torch.utils.checkpoint import checkpoint
 
-from .autograd import Operator, linear_solve
+from . import _lib as M
+from .autograd import Operator, linear_solve, native_fields
 
 E_CHARGE = 1.602176634e-19
 EPS0 = 8.8541878128e-12
@@ -84,9 +86,17 @@ class Reaction:
         return self.rate(eps_bar) if callable(self.rate) else self.rate
 
 
+class _Arrhenius:
+    def __init__(self, A, Ea):
+        self.A, self.Ea = A, Ea
+
+    def __call__(self, eps):
+        return self.A * torch.exp(-self.Ea / eps)
+
+
 def arrhenius(A, Ea):
     """k(eps) = A exp(-Ea / eps) (A in m^3/s, Ea and eps in eV)."""
-    return lambda eps: A * torch.exp(-Ea / eps)
+    return _Arrhenius(A, Ea)
 
 
 def plate_electrodes(nx, ny, device):
@@ -228,9 +238,98 @@ class Discharge:
         return torch.cat([q[:1], z, q[-1:]], dim=0)
 
     # ------------------------------------------------------------ one step
+    # the methods whose work the native step does in its own passes
+    _PIECES = frozenset(("potential", "efield", "mean_energy", "rates", "thermal_outflow", "solve_species",
+                         "solve_energy"))
+
+    def _native(self, dens, neps, V):
+        """The library's description of this step, or None where the step is
+        to be built from tensor operations: where a gradient is wanted, a
+        method is replaced, a rate is a function of the caller's, or a field
+        is not a plain contiguous one of the model's shape on the current
+        GPU."""
+        if type(self) is not Discharge or not self._PIECES.isdisjoint(self.__dict__) or self.dev.type != "cuda":
+            return None
+        ns, nr, nz = len(self.species), len(self.reactions), self.shape[0]
+        num = (int, float)
+        if ns > M.DIS_SPECIES or nr > M.DIS_REACTIONS or nz < 2 or len(dens) != ns or len(set(self.names)) != ns:
+            return None
+        fields = tuple(dens) + ((neps,) if self.energy else ())
+        if not native_fields(self.shape, self.eps_r, *fields):
+            return None
+        if torch.is_grad_enabled() and any(t.requires_grad for t in (self.eps_r,) + fields):
+            return None
+        d = M.Discharge()
+        d.nspecies, d.nreactions, d.energy, d.electron = ns, nr, int(self.energy), -1
+        scalars = [self.dt, self.h, self.Ng, self.Tg_eV, *self.eps_lfa]
+        for k, s in enumerate(self.species):
+            scalars += [s.charge, s.mu, s.mass]
+            if s.name != self.names[k] or not all(isinstance(v, num) for v in scalars):
+                return None
+            d.charge[k] = s.charge
+            d.dens[k] = dens[k].data_ptr()
+            if s.name == "e":
+                d.electron = k
+                d.cbar_num, d.cbar_den = 8.0 * E_CHARGE, math.pi * s.mass
+            if s.electrode == "FLUX":
+                d.outflow[k] = 1
+                if s.name != "e":
+                    d.cbar[k] = math.sqrt(8.0 * E_CHARGE * self.Tg_eV / (math.pi * s.mass))
+        for r, re in enumerate(self.reactions):
+            arr = type(re.rate) is _Arrhenius
+            if type(re) is not Reaction:
+                return None
+            rate, ea = (re.rate.A, re.rate.Ea) if arr else (re.rate, 0.0)
+            if not all(isinstance(v, num) for v in (rate, ea, re.energy)) or len(re.reactants) > M.DIS_ORDER:
+                return None
+            d.arrhenius[r], d.rate[r], d.ea[r], d.loss[r], d.order[r] = arr, rate, ea, re.energy, len(re.reactants)
+            for m, name in enumerate(re.reactants):
+                if name != "gas" and name not in self.names:
+                    return None
+                # ("gas" is the background also where a species has that name)
+                d.reactant[r][m] = -1 if name == "gas" else self.names.index(name)
+            for k, name in enumerate(self.names):
+                d.nu[k][r] = re.products.count(name) - re.reactants.count(name)
+        lo, hi = self.faces(V)
+        if not native_fields(self.shape[1:], lo, hi) or torch.is_grad_enabled() and (lo.requires_grad or
+                                                                                     hi.requires_grad):
+            return None
+        d.rho_coef, d.wall_weight = E_CHARGE / EPS0, 2.0 / (self.h * self.h)
+        d.dt, d.h, d.gas, d.T_gas, (d.eps0, d.eps_ref) = self.dt, self.h, self.Ng, self.Tg_eV, self.eps_lfa
+        if self.energy:
+            e = self.species[d.electron]
+            d.neps, d.mu_e = neps.data_ptr(), e.mu
+            d.elastic = 3.0 * (M_E / M_AR) * (E_CHARGE / (M_E * e.mu))
+        d.eps_r, d.lo, d.hi = self.eps_r.data_ptr(), lo.data_ptr(), hi.data_ptr()
+        return d, (lo, hi)
+
+    def _native_step(self, d, dens, neps):
+        lib, nzyx = M.load(), self.shape
+        n = nzyx[::-1]
+        new = lambda *lead: torch.empty(lead + nzyx, dtype=torch.float64, device=self.dev)  # noqa: E731
+        stream = torch.cuda.current_stream().cuda_stream
+        charge, E, rhs = new(), new(3), new(d.nspecies + d.energy)
+        M.check(lib.mps_charge_rhs(stream, *n, d, charge.data_ptr()))
+        phi = self.solve_poisson(charge)
+        d.phi, d.E, d.rhs = phi.data_ptr(), E.data_ptr(), rhs.data_ptr()
+        M.check(lib.mps_discharge_rhs(stream, *n, d))
+        out = []
+        for k, (s, nsp) in enumerate(zip(self.species, dens)):
+            drift = s.charge != 0 and s.mu > 0
+            out.append(self.ops[k].advance(rhs[k], nsp, tuple(E) if drift else None,
+                                           math.copysign(s.mu, s.charge) if drift else 1.0))
+        if not self.energy:
+            return tuple(out), None
+        ve = -(5.0 / 3.0) * self.species[d.electron].mu
+        return tuple(out), self.energy_op.advance(rhs[-1], neps, tuple(E), ve)
+
     def step(self, dens, neps, V):
         """dens: tuple of species densities; neps: electron energy density
         (or None). Returns the new (dens, neps)."""
+        native = self._native(dens, neps, V)
+        if native is not None:
+            d, _faces = native  # (the plates' potentials live as long as d's addresses)
+            return self._native_step(d, dens, neps)
         phi = self.potential(dens, V)
         ex, ey, ez = self.efield(phi, V)
         e2 = ex * ex + ey * ey + ez * ez

@@ -1,0 +1,124 @@
+"""The library's field passes of a discharge step (mps_pad_fields,
+mps_charge_rhs, mps_discharge_rhs) against the step built from tensor
+operations: the right-hand sides and velocities that reach each solve. The
+passes do the same operations in the same order without contraction, so the
+bar is 1e-14 relative to the largest value (exp may differ by an ulp), and
+bitwise for the padded fields. Where a step may not take the passes it does
+not: gradients wanted, replaced methods, rates of the caller's, other
+layouts."""
+import pytest
+import torch
+
+from mps3d_amd import autograd as AG
+from mps3d_amd import discharge as DS
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+
+
+class Torch(DS.Discharge):
+    """A subclass: its steps are built from tensor operations."""
+
+
+def record(model):
+    """Replaces the operators' solves; returns what they are given."""
+    seen = []
+
+    class Op:
+        def __init__(self, scale):
+            self.scale = scale
+
+        def configure(self, vel=None, rhs=None, scale=1.0):
+            vg = [] if vel is None else AG.pad_fields(vel, scale)
+            seen.append([rhs.clone()] + [v.clone() for v in vg])
+            self.rhs = rhs
+
+        def solve(self, x0=None):
+            return AG.pad(self.scale * self.rhs)
+
+        advance = AG.Operator.advance
+
+        def close(self):
+            pass
+
+    model.poisson = Op(1e-9 * model.h ** 2)
+    model.ops = [Op(0.9 * model.dt) for _ in model.species]
+    if model.energy:
+        model.energy_op = Op(0.9 * model.dt)
+    return seen
+
+
+def build(cls, form, n):
+    sp = [DS.Species("e", -1, 20.0, 100.0, mass=DS.M_E), DS.Species("A+", 1, 0.2, 0.01),
+          DS.Species("A-", -1, 0.2, 0.01, electrode="ZGRD"), DS.Species("A*", 0, 0.0, 0.01)]
+    re = [DS.Reaction(("e", "gas"), ("e", "e", "A+"), DS.arrhenius(1e-13, 15.0), energy=15.0),
+          DS.Reaction(("A-", "A*"), ("e",), 1e-16), DS.Reaction(("gas",), ("A*",), 2.0),
+          DS.Reaction(("e", "A+", "gas"), ("A*",), DS.arrhenius(3e-30, 1.0), energy=-2.0)]
+    if form == "one":
+        sp, re = sp[1:2], []
+    el = DS.split_electrodes(n, n, "cuda") if form != "energy" else DS.plate_electrodes(n, n, "cuda")
+    eps = 1.0 + torch.rand((n,) * 3, dtype=F64, generator=torch.Generator().manual_seed(3))
+    return cls(n, 0.02, sp, re, el, energy=form == "energy", eps_r=eps)
+
+
+def state(model, n):
+    g = torch.Generator().manual_seed(n)
+    f = [(1e12 + 1e16 * torch.rand((n,) * 3, dtype=F64, generator=g)).cuda() for _ in range(len(model.species) + 1)]
+    return tuple(f[:-1]), (3.0 * f[-1] if model.energy else None)
+
+
+@pytest.mark.parametrize("n", [4, 6, 17, 64, 65, 70])
+@pytest.mark.parametrize("form", ["energy", "local", "one"])
+def test_passes_equal_the_tensor_operations(gpu, n, form):
+    out = []
+    V = torch.tensor([800.0, -300.0], dtype=F64, device="cuda")
+    for cls in (DS.Discharge, Torch):
+        m = build(cls, form, n)
+        solvers = [o for o in [m.poisson, *m.ops, getattr(m, "energy_op", None)] if o is not None]
+        seen = record(m)
+        dens, neps = state(m, n)
+        assert (m._native(dens, neps, V) is not None) == (cls is DS.Discharge)
+        for _ in range(2):
+            new, neps = m.step(dens, neps, V)
+            dens = tuple(d.clone() for d in new)
+        out.append(seen)
+        for o in solvers:
+            o.close()
+    assert len(out[0]) == len(out[1])
+    for a, b in zip(*out):
+        assert len(a) == len(b)
+        for x, y in zip(a, b):
+            assert float((x - y).abs().max()) <= 1e-14 * float(y.abs().max())
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 4, 5), (2, 9, 63), (5, 3, 64), (4, 8, 131)])
+def test_pad_fields(gpu, shape):
+    f = [torch.randn(shape, dtype=F64, device="cuda") for _ in range(4)]
+    for k in (1, 3, 4):
+        for s in (1.0, -0.3):
+            for got, t in zip(AG.pad_fields(f[:k], s), f[:k]):
+                assert torch.equal(got, AG.pad(s * t))
+    t = torch.randn(shape[::-1], dtype=F64, device="cuda").permute(2, 1, 0)   # not contiguous: tensor operations
+    assert torch.equal(AG.pad_fields([t])[0], AG.pad(t))
+    assert AG.pad_fields([f[0].float()])[0].dtype == torch.float32
+
+
+def test_steps_that_stay_tensor_operations(gpu):
+    m = build(DS.Discharge, "energy", 6)
+    dens, neps = state(m, 6)
+    V = torch.tensor([800.0], dtype=F64, device="cuda")
+    assert m._native(dens, neps, V) is not None
+    Vg = V.clone().requires_grad_()
+    assert m._native(dens, neps, Vg) is None
+    assert m._native((dens[0].clone().requires_grad_(),) + dens[1:], neps, V) is None
+    with torch.no_grad():
+        assert m._native(dens, neps, Vg) is not None
+    assert m._native((dens[0].permute(2, 1, 0),) + dens[1:], neps, V) is None
+    with torch.autograd.forward_ad.dual_level():
+        assert m._native(dens, neps, V) is None
+    m.solve_species = lambda k, rhs, vel, x0: rhs
+    assert m._native(dens, neps, V) is None
+    del m.solve_species
+    m.reactions[0].rate = lambda eps: 1e-13 * torch.exp(-15.0 / eps)
+    assert m._native(dens, neps, V) is None
+    m.close()
