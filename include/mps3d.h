@@ -529,6 +529,12 @@ int mps_discharge_rhs(void *stream, int nx, int ny, int nz, const mps_discharge 
  * against it. */
 void *mps_stream(mps_ctx *ctx);
 
+/* Every call orders the context's stream after the null stream. hold = 1
+ * does that once, now, and the calls until hold = 0 don't: for a row of calls
+ * on one context with no other device work between them (an event recorded
+ * and waited for costs the host about 15 us). */
+int mps_hold_order(mps_ctx *ctx, int hold);
+
 const char *mps_error_string(int status);
 /* Text of the most recent failure on this thread. */
 const char *mps_last_error(void);

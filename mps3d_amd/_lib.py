@@ -34,7 +34,7 @@ EXPORTS = (
     "mps_time_in_solve",
     "mps_get_grid", "mps_gmres_noalloc", "mps_restrict", "mps_prolong1",
     "mps_eden_faces", "mps_neutral_faces", "mps_eenergy_faces", "mps_floor", "mps_set_source",
-    "mps_pad_fields", "mps_charge_rhs", "mps_discharge_rhs",
+    "mps_pad_fields", "mps_charge_rhs", "mps_discharge_rhs", "mps_hold_order",
 )
 # sizes of mps_pad_fields and mps_discharge
 PAD_FIELDS, DIS_SPECIES, DIS_REACTIONS, DIS_ORDER = 4, 8, 8, 4
@@ -137,6 +137,7 @@ def load():
     L.mps_eenergy_faces.argtypes = [_vp, C.POINTER(C.c_int), _vp, _vp, C.c_double, _vp, C.c_double, _vp]
     L.mps_floor.argtypes = [_vp, _vp, C.c_double]
     L.mps_set_source.argtypes = [_vp, _vp]
+    L.mps_hold_order.argtypes = [_vp, C.c_int]
     L.mps_pad_fields.argtypes = [_vp] + [C.c_int] * 4 + [C.POINTER(_vp), C.c_double, _vp]
     L.mps_charge_rhs.argtypes = [_vp] + [C.c_int] * 3 + [C.POINTER(Discharge), _vp]
     L.mps_discharge_rhs.argtypes = [_vp] + [C.c_int] * 3 + [C.POINTER(Discharge)]

@@ -198,6 +198,7 @@ struct mps_ctx {
     double *user_tmp2 = nullptr;         // staging for interior arrays
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t ev_in = nullptr;          // orders calls after the null stream
+    bool hold_order = false;             // (not while held: mps_hold_order)
     hipEvent_t ev_inv = nullptr;         // the coarsest inverse's status has been copied
     bool inv_pending = false;            // and set_coeffs has yet to read it
     bool tail_dirty = true;              // coefficients or BC codes changed since k_tail_rows
@@ -1572,6 +1573,7 @@ struct ExactScope {
 // arrays produced there are complete before this call reads them.
 int after_null_stream(mps_ctx *c)
 {
+    if (c->hold_order) return MPS_OK;
     hipError_t e = hipEventRecord(c->ev_in, nullptr);
     if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, c->ev_in, 0);
     if (e != hipSuccess) return fail(MPS_ERR_HIP, "ordering after the null stream: %s", hipGetErrorString(e));
@@ -2136,6 +2138,15 @@ const char *mps_error_string(int s)
 const char *mps_last_error(void) { return g_last_error.c_str(); }
 
 void *mps_stream(mps_ctx *c) { return c ? (void *)c->stream : nullptr; }
+
+int mps_hold_order(mps_ctx *c, int hold)
+{
+    if (!c) return fail(MPS_ERR_ARG, "null context");
+    c->hold_order = false;
+    const int st = hold ? guard(c, false) : MPS_OK;
+    c->hold_order = hold != 0 && st == MPS_OK;
+    return st;
+}
 
 int mps_destroy(mps_ctx *c)
 {

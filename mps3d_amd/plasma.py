@@ -188,6 +188,12 @@ class PlasmaRun:
                      for _ in self.neutrals],
             "ener": [self._face_full(f, 0.0) for f in FACES],
         }
+        # the transport coefficients of each context (rewritten by each call)
+        nul = lambda m: self.eprod.new_zeros(m * self.eprod.numel())  # noqa: E731
+        self._out = {q: {"vel": nul(3), "dcoeff": nul(1), "reac": nul(1), "source": nul(1), "prod": None}
+                     for q in ("pois", "ener", "elec", "ion") + (("neut",) if self.neutrals else ())}
+        self._out["ion"]["prod"] = nul(1)
+        self._still = nul(3) if self.neutrals else None
         self.t = 0.0
         self.steps = 0
         self.cycles = []
@@ -236,54 +242,67 @@ class PlasmaRun:
         e = ch.especnum - 1
         dt_s = self.dt / self.t0
         cyc = []
+        # Each equation is one row of calls on its context: the transport's
+        # coefficients go into arrays kept for the context, and torch works
+        # between the rows only.
         # poisson_solve (poissoneq.f90:387-470); the potential's faces stay
         # (poisson_update_bcs changes only 'DZGD' electrodes)
         ions = self.numden[self.ions[0]:self.ions[-1] + 1].reshape(-1)
-        co = self.pois.poisson_transport(self.numden[e].reshape(-1), ions, self.scal["pot"], timederiv=False, dt=dt_s)
-        # (its coefficients never change: the permittivity-free operator
-        # dcoeff = tscale/lscale^2 of poisson_update_transport; only the source)
-        cyc.append(self._solve(self.pois, self.phi_s, self.codes["pot"], self.faces["pot"], co, False, dt_s,
-                               faces_changed=self.steps == 0, coeffs_changed=self.steps == 0))
+        with self.pois.chained():
+            co = self.pois.poisson_transport(self.numden[e].reshape(-1), ions, self.scal["pot"], timederiv=False,
+                                             dt=dt_s, out=self._out["pois"])
+            # (its coefficients never change: the permittivity-free operator
+            # dcoeff = tscale/lscale^2 of poisson_update_transport; only the source)
+            cyc.append(self._solve(self.pois, self.phi_s, self.codes["pot"], self.faces["pot"], co, False, dt_s,
+                                   faces_changed=self.steps == 0, coeffs_changed=self.steps == 0))
+            # update_efield (poissoneq.f90:565-680)
+            self.pois.efield(self.phi_s, self.potscale / self.L0, False, out=self.E)
         self.pot = self.phi_s * self.potscale
-        # update_efield (poissoneq.f90:565-680)
-        self.pois.efield(self.phi_s, self.potscale / self.L0, False, out=self.E)
         # eenergy_solve (eenergyeq.f90:776-840) and update_electrontemp
-        co = self.ener.eenergy_transport(self.E.reshape(-1), self.Te.reshape(-1), self.numden.reshape(-1),
-                                         self.scal["ener"], lscale=self.L0, soln=self.eps_s.reshape(-1),
-                                         dt=dt_s, Tg=self.Tg, Pg=self.Pg)
-        self._eenergy_bcs()
-        cyc.append(self._solve(self.ener, self.eps_s, self.codes["etemp"], self.faces["ener"], co, True, dt_s))
-        self.ener.electron_temp(self.eps_s, self.numden[e], self.eescale, self.etempmin, self.Te)
+        with self.ener.chained():
+            co = self.ener.eenergy_transport(self.E.reshape(-1), self.Te.reshape(-1), self.numden.reshape(-1),
+                                             self.scal["ener"], lscale=self.L0, soln=self.eps_s.reshape(-1),
+                                             dt=dt_s, Tg=self.Tg, Pg=self.Pg, out=self._out["ener"])
+            self._eenergy_bcs()
+            cyc.append(self._solve(self.ener, self.eps_s, self.codes["etemp"], self.faces["ener"], co, True, dt_s))
+            self.ener.electron_temp(self.eps_s, self.numden[e], self.eescale, self.etempmin, self.Te)
         self.eps = self.eps_s * self.eescale
         # eden_solve (edeneq.f90:446-523)
-        co = self.elec.species_transport(ch.especnum, self.E.reshape(-1), self.Te.reshape(-1),
-                                         self.numden.reshape(-1), self.scal["eden"], soln=self.ne_s.reshape(-1),
-                                         dt=dt_s, Tg=self.Tg, Pg=self.Pg, out={"prod": self.eprod.view(-1)})
-        self._eden_bcs()
-        cyc.append(self._solve(self.elec, self.ne_s, self.codes["eden"], self.faces["eden"], co, True, dt_s))
-        self.elec.floor(self.ne_s, self.nemin)
+        with self.elec.chained():
+            co = self.elec.species_transport(ch.especnum, self.E.reshape(-1), self.Te.reshape(-1),
+                                             self.numden.reshape(-1), self.scal["eden"], soln=self.ne_s.reshape(-1),
+                                             dt=dt_s, Tg=self.Tg, Pg=self.Pg,
+                                             out=dict(self._out["elec"], prod=self.eprod.view(-1)))
+            self._eden_bcs()
+            cyc.append(self._solve(self.elec, self.ne_s, self.codes["eden"], self.faces["eden"], co, True, dt_s))
+            self.elec.floor(self.ne_s, self.nemin)
         self.numden[e].copy_(self.ne_s * self.escale_n)
         # ions_solve (ionseq.f90:560-629): every ion from the same densities,
         # which take the new ion densities after the last one
         for q, sp in enumerate(self.ions):
-            co = self.ion.species_transport(sp + 1, self.E.reshape(-1), self.Te.reshape(-1),
-                                            self.numden.reshape(-1), self.scal["ion"],
-                                            soln=self.ni_s[q].reshape(-1), dt=dt_s, Tg=self.Tg, Pg=self.Pg)
-            self._ion_bcs(q, sp)
-            cyc.append(self._solve(self.ion, self.ni_s[q], self.codes["spec"], self.faces["ion"][q], co, True, dt_s))
+            flux = self._ion_faces(q)
+            with self.ion.chained():
+                co = self.ion.species_transport(sp + 1, self.E.reshape(-1), self.Te.reshape(-1),
+                                                self.numden.reshape(-1), self.scal["ion"],
+                                                soln=self.ni_s[q].reshape(-1), dt=dt_s, Tg=self.Tg, Pg=self.Pg,
+                                                out=self._out["ion"])
+                self._ion_bcs(q, sp, flux)
+                cyc.append(self._solve(self.ion, self.ni_s[q], self.codes["spec"], self.faces["ion"][q], co, True,
+                                       dt_s))
         for q, sp in enumerate(self.ions):
             self.numden[sp].copy_(self.ni_s[q] * self.iscale)
         # neutrals_solve (neutralseq.f90:438-508), after it the same update
         for q, sp in enumerate(self.neutrals):
-            co = self.neut.species_transport(sp + 1, self.E.reshape(-1), self.Te.reshape(-1),
-                                             self.numden.reshape(-1), self.scal["neut"],
-                                             soln=self.nn_s[q].reshape(-1), dt=dt_s, Tg=self.Tg, Pg=self.Pg,
-                                             out={"prod": self.nprod[q].view(-1)})
-            # neutrals_update_transport leaves vel at zero
-            co["vel"].zero_()
-            self._neutral_bcs(q, sp)
-            cyc.append(self._solve(self.neut, self.nn_s[q], self.codes["spec"], self.faces["neut"][q], co, True,
-                                   dt_s))
+            with self.neut.chained():
+                co = self.neut.species_transport(sp + 1, self.E.reshape(-1), self.Te.reshape(-1),
+                                                 self.numden.reshape(-1), self.scal["neut"],
+                                                 soln=self.nn_s[q].reshape(-1), dt=dt_s, Tg=self.Tg, Pg=self.Pg,
+                                                 out=dict(self._out["neut"], prod=self.nprod[q].view(-1)))
+                # neutrals_update_transport leaves vel at zero
+                co["vel"] = self._still
+                self._neutral_bcs(q, sp)
+                cyc.append(self._solve(self.neut, self.nn_s[q], self.codes["spec"], self.faces["neut"][q], co, True,
+                                       dt_s))
         for q, sp in enumerate(self.neutrals):
             self.numden[sp].copy_(self.nn_s[q] * self.nscale)
         self.t = self.t + self.dt
@@ -310,10 +329,8 @@ class PlasmaRun:
         self.ener.eenergy_faces(self.codes["etemp"], self.eps_s.reshape(-1), ne.reshape(-1), self.eescale,
                                 self.params["etemp"], self.vel_scaling, self.faces["ener"])
 
-    def _ion_bcs(self, q, sp):
-        """ions_update_bcs (ionseq.f90:206-476) for ion sp: FLUX faces carry
-        the drift outflow mu n E_normal where it leaves the domain, else
-        zero."""
+    def _ion_faces(self, q):
+        """The FLUX faces of ion q for _ion_bcs; its DIRC faces scaled."""
         faces = self.faces["ion"][q]
         flux = [None] * 6
         for k, f in enumerate(FACES):
@@ -323,6 +340,12 @@ class PlasmaRun:
                 faces[k] = self._div(faces[k], self.iscale)
             elif code == "FLUX":
                 flux[k] = faces[k]    # rewritten in place: mps_set_bc copies the faces
+        return flux
+
+    def _ion_bcs(self, q, sp, flux):
+        """ions_update_bcs (ionseq.f90:206-476) for ion sp: FLUX faces carry
+        the drift outflow mu n E_normal where it leaves the domain, else
+        zero."""
         if any(t is not None for t in flux):
             # all FLUX faces of this ion in one launch (mps_ion_drift_faces)
             self.ion.ion_drift_faces(sp + 1, self.E.reshape(-1), self.numden.reshape(-1),

@@ -27,6 +27,8 @@ Every compute call goes to the HIP library; there is no CPU fallback.
 from __future__ import annotations
 
 import ctypes as C
+import math
+from contextlib import contextmanager
 
 import numpy as np
 
@@ -127,6 +129,7 @@ class FieldSolver:
         self._keep = []
         self._ext = None        # the context's stream as a torch ExternalStream
         self._torch_call = False
+        self._chained = False
         self._chem = None       # the Chemistry of the last set_chemistry
 
     # ------------------------------------------------------------ plumbing
@@ -151,15 +154,19 @@ class FieldSolver:
     def __exit__(self, *a):
         self.close()
 
-    def order_torch_in(self):
+    def order_torch_in(self, faces=False):
         """Orders the context's stream after torch's current stream (device-
         side, no host wait): tensors torch is still writing are complete
-        before the library reads them. The library itself only orders after
-        the null stream."""
+        before the library reads them. Every entry point that takes device
+        arrays orders after the null stream by itself, so there is nothing to
+        do here where that is torch's stream (an event recorded and waited
+        for costs the host 20 us)."""
         import torch
         if self._ext is None:
             self._ext = torch.cuda.ExternalStream(self.lib.mps_stream(self._h))
-        self._ext.wait_stream(torch.cuda.current_stream())
+        cur = torch.cuda.current_stream()
+        if cur.cuda_stream != 0 or faces:
+            self._ext.wait_stream(cur)
         self._torch_call = True
 
     def order_torch_out(self):
@@ -179,11 +186,12 @@ class FieldSolver:
             import torch
             if not a.is_cuda or a.dtype != torch.float64 or not a.is_contiguous():
                 raise ValueError("device arrays must be contiguous float64 tensors on the GPU")
-            want = {"g": int(np.prod(self.shape)), "i": int(np.prod(self.n))}.get(kind)
+            want = math.prod(self.shape) if kind == "g" else math.prod(self.n) if kind == "i" else None
             if want is not None and a.numel() != want:
                 raise ValueError("device array has %d elements, expected %d" % (a.numel(), want))
             if not self._torch_call:
-                self.order_torch_in()
+                # (mps_set_bc reads faces of a mixed set with the host's copies)
+                self.order_torch_in(kind == "f")
             return C.c_void_p(a.data_ptr())
         arr = np.asarray(a, dtype=np.float64)
         if kind == "g":
@@ -204,7 +212,23 @@ class FieldSolver:
 
     def _release(self):
         self._keep = []
-        if self._torch_call:
+        if self._torch_call and not self._chained:
+            self.order_torch_out()
+
+    @contextmanager
+    def chained(self):
+        """A row of calls on this context with no torch operation between
+        them: ordered after torch's stream once, before the first, and torch's
+        stream after them once, at the end (each of the two costs the host
+        about 20 us a call)."""
+        self.order_torch_in()
+        try:
+            M.check(self.lib.mps_hold_order(self._h, 1))
+            self._chained = True
+            yield
+        finally:
+            self._chained = False
+            self.lib.mps_hold_order(self._h, 0)
             self.order_torch_out()
 
     # ------------------------------------------------------------ set-up
@@ -290,7 +314,7 @@ class FieldSolver:
         E = out if out is not None else np.zeros((nx + 2, ny + 2, nz + 2, 3), order="F")
         try:
             if _is_torch(E):
-                if E.numel() != 3 * int(np.prod(self.shape)):
+                if E.numel() != 3 * math.prod(self.shape):
                     raise ValueError("efield needs 3 ghosted components")
                 ep = self._ptr(E, None, True)
             else:
@@ -308,7 +332,7 @@ class FieldSolver:
         be Fortran-ordered float64)."""
         if a is None:
             return None
-        want = ncomp * int(np.prod(self.shape))
+        want = ncomp * math.prod(self.shape)
         if _is_torch(a):
             import torch
             if not a.is_cuda or a.dtype != torch.float64 or not a.is_contiguous() or a.numel() != want:
@@ -335,7 +359,7 @@ class FieldSolver:
         res = dict(out or {})
         if device:
             import torch
-            ng = int(np.prod(g))
+            ng = math.prod(g)
             dev = device
             for k, m in (("vel", 3), ("dcoeff", 1), ("reac", 1), ("source", 1), ("prod", 1)):
                 if k not in res:
