@@ -156,10 +156,10 @@ struct GmresBufs {
     int m = 0;
     std::vector<double *> V, Z;
     double *w = nullptr, *bg = nullptr, *dh = nullptr, *dpart = nullptr;
-    double *hh = nullptr;  // pinned host mirror of dh
+    double *hh = nullptr;  // pinned: the first norms
     int nblocks = 0;
     // device Arnoldi state: H, cs, sn, gv, y, hn, the second Gram-Schmidt
-    // pass's products h2, the subtracted coefficients ny and |w|^2
+    // pass's products h2 and the subtracted coefficients ny
     double *darn = nullptr;
     int *dstate = nullptr;
     int *hflag = nullptr;                // pinned: per step the done flag, then kk and the NaN flag
@@ -256,6 +256,15 @@ dim3 colour_grid(const Geom &g)
 dim3 red_grid(const Geom &g)
 {
     return dim3((unsigned)((g.nx * g.ny + kBlock - 1) / kBlock), (unsigned)std::min(g.nz, 16));
+}
+// reductions that apply the operator: more, shorter k loops, enough blocks to
+// hide the latency of its fifteen reads (an SG residual at 129^3: 44 us with 16
+// planes of blocks, 38 with 31)
+dim3 red_rows_grid(const Geom &g)
+{
+    dim3 gr = red_grid(g);
+    gr.y = (unsigned)std::min(g.nz, std::max(16, (int)(4096 / gr.x)));
+    return gr;
 }
 dim3 block() { return dim3(kBlock); }
 
@@ -796,7 +805,7 @@ void launch_prolong_tri(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l)
 int residual_max_partials(const Geom &g)
 {
     int kz;
-    dim3 a = residual_planes_grid(g, kz), b = red_grid(g);
+    dim3 a = residual_planes_grid(g, kz), b = red_rows_grid(g);
     return (int)std::max(a.x * a.y * a.z, b.x * b.y);
 }
 
@@ -827,7 +836,7 @@ int launch_residual(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, const T *u, 
         }
         return partials ? (int)(gr.x * gr.y * gr.z) : 0;
     }
-    const dim3 gr = (reduce_grid || partials) ? red_grid(g) : cells_grid(g);
+    const dim3 gr = (reduce_grid || partials) ? red_rows_grid(g) : cells_grid(g);
     with_op(op, c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
         hipLaunchKernelGGL((k_residual<T, R_, decltype(O)::value, decltype(V)::value, decltype(R)::value>), gr,
                            block(), 0, c->stream, v, u, b, r, partials, rscale);
@@ -3489,52 +3498,47 @@ void release_weights(mps_ctx *c)
         for (int d = 0; d < 3; ++d) c->LT[l].w[d] = nullptr;
 }
 
-// one V-cycle preconditioner application z = M^-1 v (homogeneous BCs,
-// zero initial guess), in FP64 or with FP32 inner cycles
-void precondition(mps_ctx *c, const double *v, double *z)
+// One V-cycle preconditioner application from a zero guess (homogeneous BCs)
+// and w = A M^-1 v with w's products with the first min(nv, kDotRegs) of vs
+// left in out: z = M^-1 v. With FP32 inner cycles v is in the finest level's
+// FP32 right-hand side (k_scale put it there) and the operator reads the
+// cycle's FP32 correction.
+void precondition_matvec(mps_ctx *c, GmresBufs &G, const double *v, double *z, double *w, double *const *vs, int nv,
+                         double *out)
 {
     const Geom &g = c->geom[0];
+    VecList VL{};
+    for (int q = 0; q < nv; ++q) VL.v[q] = vs[q];
+    const int nd = std::min(nv, kDotRegs);
+    const dim3 gr = red_rows_grid(g);
+    auto product = [&](auto *u) {
+        Lev<double> l0 = view(c, c->L64, 0);
+        with_op(level_op(c, c->L64, 0), c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
+            using U = std::remove_const_t<std::remove_pointer_t<decltype(u)>>;
+            hipLaunchKernelGGL((k_matvec_dots<U, decltype(O)::value, decltype(V)::value, decltype(R)::value>), gr,
+                               block(), 0, c->stream, l0, u, z, w, VL, nd, G.dpart);
+        });
+    };
     if (c->opts.precision == MPS_PREC_FP32_DC) {
         auto &F = c->L32;
-        convert<double, float>(c, v, F[0].b, g.ng());
-        fill<float>(c, F[0].u, g.ng(), 0.0f);
-        vcycle<float>(c, F, 0, c->bottom32, true);
-        convert<float, double>(c, F[0].u, z, g.ng());
+        vcycle<float>(c, F, 0, c->bottom32, true, true);
+        product((const float *)F[0].u);
     } else {
         auto &L = c->L64;
-        fill<double>(c, z, g.ng(), 0.0);
         double *ub = L[0].u, *bb = L[0].b;
         L[0].u = z;
         L[0].b = const_cast<double *>(v);
-        vcycle<double>(c, L, 0, c->bottom64, true);
+        vcycle<double>(c, L, 0, c->bottom64, true, true);
+        z = L[0].u;
         L[0].u = ub;
         L[0].b = bb;
+        product((const double *)z);
     }
+    hipLaunchKernelGGL(k_reduce_cols, dim3(nd), block(), 0, c->stream, (const double *)G.dpart, (int)(gr.x * gr.y),
+                       out);
 }
 
-void matvec(mps_ctx *c, std::vector<LevelBuf<double>> &L, const double *u, double *out)
-{
-    Lev<double> v = view(c, L, 0);
-    with_op(level_op(c, L, 0), c->has_vel, c->has_reac, [&](auto O, auto V, auto R) {
-        hipLaunchKernelGGL((k_matvec<double, decltype(O)::value, decltype(V)::value, decltype(R)::value>),
-                           cells_grid(c->geom[0]), block(), 0, c->stream, v, u, out);
-    });
-}
-
-// sum_q of (w . v_q) for q < nv into host h[0..nv)
-void multidot(mps_ctx *c, GmresBufs &G, const double *w, double *const *vs, int nv, double *h)
-{
-    Lev<double> v = view(c, c->L64, 0);
-    VecList VL{};
-    for (int q = 0; q < nv; ++q) VL.v[q] = vs[q];
-    hipLaunchKernelGGL(k_multidot, red_grid(c->geom[0]), block(), 0, c->stream, v, w, VL, nv, G.dpart);
-    hipLaunchKernelGGL(k_reduce_cols, dim3(nv), block(), 0, c->stream, (const double *)G.dpart, G.nblocks, G.dh);
-    HIPCHK(hipMemcpyAsync(G.hh, G.dh, nv * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    std::memcpy(h, G.hh, nv * sizeof(double));
-}
-
-// multidot with the products left on the device in out[0..nv)
+// w . v_q for q < nv into out[0..nv) (device)
 void multidot_dev(mps_ctx *c, GmresBufs &G, const double *w, double *const *vs, int nv, double *out)
 {
     Lev<double> v = view(c, c->L64, 0);
@@ -3545,18 +3549,29 @@ void multidot_dev(mps_ctx *c, GmresBufs &G, const double *w, double *const *vs, 
 }
 
 // w -= sum_q h[q] v_q with device coefficients h (the first min(nv, *nvd)
-// when nvd is given); |w|^2 into *norm2 (device) when norm2 is given
-void multiaxpy_dev(mps_ctx *c, double *w, double *const *vs, int nv, const double *h, const int *nvd,
-                   double *norm2)
+// when nvd is given), with block partials of |w|^2 in c->partials (their
+// number is returned)
+int multiaxpy_dev(mps_ctx *c, double *w, double *const *vs, int nv, const double *h, const int *nvd)
 {
     Lev<double> v = view(c, c->L64, 0);
     VecList VL{};
     for (int q = 0; q < nv; ++q) VL.v[q] = vs[q];
     dim3 gr = red_grid(c->geom[0]);
-    hipLaunchKernelGGL(k_multiaxpy, gr, block(), 0, c->stream, v, w, VL, h, nv, norm2 ? c->partials : nullptr, nvd);
-    if (norm2)
-        hipLaunchKernelGGL(k_reduce_final, dim3(1), block(), 0, c->stream, (const double *)c->partials,
-                           (int)(gr.x * gr.y), norm2);
+    hipLaunchKernelGGL(k_multiaxpy, gr, block(), 0, c->stream, v, w, VL, h, nv, c->partials, nvd);
+    return (int)(gr.x * gr.y);
+}
+
+// the same, and the new w's products with vs into out
+void multiaxpy_dots(mps_ctx *c, GmresBufs &G, double *w, double *const *vs, int nv, const double *h, double *out)
+{
+    Lev<double> v = view(c, c->L64, 0);
+    VecList VL{};
+    for (int q = 0; q < nv; ++q) VL.v[q] = vs[q];
+    const dim3 gr = red_grid(c->geom[0]);
+    hipLaunchKernelGGL(k_multiaxpy_dots, gr, block(), 0, c->stream, v, w, VL, h, nv, G.dpart);
+    hipLaunchKernelGGL(k_reduce_cols, dim3(std::min(nv, kDotRegs)), block(), 0, c->stream, (const double *)G.dpart,
+                       (int)(gr.x * gr.y), out);
+    if (nv > kDotRegs) multidot_dev(c, G, w, vs + kDotRegs, nv - kDotRegs, out + kDotRegs);
 }
 
 // performgmres with the reference's preconditioner on the finest level (at
@@ -3604,7 +3619,7 @@ void free_gmres(GmresBufs &G)
 // sizes of the device Arnoldi block (doubles) for m <= kMaxVec - 1
 constexpr int kArnLd = kMaxVec;                    // leading dimension of H (m + 1 <= kMaxVec)
 constexpr size_t kArnH = (size_t)kArnLd * kMaxVec; // H
-constexpr size_t kArnDoubles = kArnH + 7 * (size_t)kMaxVec + 1;
+constexpr size_t kArnDoubles = kArnH + 7 * (size_t)kMaxVec;
 
 ArnoldiDev arnoldi_view(GmresBufs &G)
 {
@@ -3619,10 +3634,9 @@ ArnoldiDev arnoldi_view(GmresBufs &G)
     A.state = G.dstate;
     return A;
 }
-// the second pass's products, the subtracted coefficients and |w|^2
+// the second pass's products and the subtracted coefficients
 double *arn_h2(GmresBufs &G) { return G.darn + kArnH + 5 * (size_t)kMaxVec; }
 double *arn_ny(GmresBufs &G) { return G.darn + kArnH + 6 * (size_t)kMaxVec; }
-double *arn_wn2(GmresBufs &G) { return G.darn + kArnH + 7 * (size_t)kMaxVec; }
 
 // the context's FGMRES(m) vectors, (re)allocated when m grows. Every vector
 // starts with zero ghosts and the Krylov kernels write interiors only, so
@@ -3641,7 +3655,8 @@ GmresBufs &gmres_bufs(mps_ctx *c, int m)
     G.w = dalloc<double>(g.ng());
     G.bg = dalloc<double>(g.ng());
     G.dh = dalloc<double>(kMaxVec);
-    G.dpart = dalloc<double>((size_t)G.nblocks * kMaxVec);
+    const dim3 rr = red_rows_grid(g);
+    G.dpart = dalloc<double>(std::max((size_t)G.nblocks * kMaxVec, (size_t)rr.x * rr.y * kDotRegs));
     HIPCHK(hipHostMalloc((void **)&G.hh, kMaxVec * sizeof(double), hipHostMallocDefault));
     G.darn = dalloc<double>(kArnDoubles);
     G.dstate = dalloc<int>(4);
@@ -3657,11 +3672,13 @@ GmresBufs &gmres_bufs(mps_ctx *c, int m)
     return G;
 }
 
-// v = w / s[0] with s on the device (nothing when s[0] <= 0)
+// v = w / s[0] with s on the device (nothing when s[0] <= 0), and, with FP32
+// inner cycles, the next cycle's right-hand side
 void scale_from(mps_ctx *c, const double *w, double *v, const double *s)
 {
     Lev<double> vw = view(c, c->L64, 0);
-    hipLaunchKernelGGL(k_scale, cells_grid(c->geom[0]), block(), 0, c->stream, vw, w, v, s);
+    float *f = c->opts.precision == MPS_PREC_FP32_DC ? c->L32[0].b : nullptr;
+    hipLaunchKernelGGL(k_scale, cells_grid(c->geom[0]), block(), 0, c->stream, vw, w, v, s, f);
 }
 
 }  // namespace
@@ -3705,21 +3722,25 @@ int mps_gmres(mps_ctx *c, const double *b, double *x, int m, int max_restarts, d
         GmresBufs &G = gmres_bufs(c, m);
         const double *bd = stage_interior(c, b);
         Lev<double> v0 = view(c, c->L64, 0);
-        hipLaunchKernelGGL(k_interior_in<double>, cells_grid(g), block(), 0, c->stream, v0, bd, G.bg);
-        double bn2;
-        {
-            double *one[1] = {G.bg};
-            multidot(c, G, G.bg, one, 1, &bn2);
-        }
-        const double bnorm = std::sqrt(bn2);
+        const dim3 rg = red_grid(g);
+        hipLaunchKernelGGL(k_interior_in_sq, rg, block(), 0, c->stream, v0, bd, G.bg, G.dpart);
+        auto residual = [&]() {  // w = b - A x; the number of partials of |w|^2
+            return launch_residual<double, double>(c, c->L64, 0, u, G.bg, G.w, c->partials, level_op(c, 0));
+        };
         auto true_residual = [&]() {  // w = b - A x, returns ||w||
-            const int np = launch_residual<double, double>(c, c->L64, 0, u, G.bg, G.w, c->partials, level_op(c, 0));
+            const int np = residual();
             hipLaunchKernelGGL(k_reduce_final, dim3(1), block(), 0, c->stream, (const double *)c->partials, np,
                                c->d_scalar);
             return std::sqrt(read_scalar(c));
         };
+        const int np0 = residual();
+        hipLaunchKernelGGL(k_reduce_pair, dim3(2), block(), 0, c->stream, (const double *)c->partials, np0,
+                           (const double *)G.dpart, (int)(rg.x * rg.y), c->d_scalar);
+        HIPCHK(hipMemcpyAsync(G.hh, c->d_scalar, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        const double bnorm = std::sqrt(G.hh[1]);
         int total = 0;
-        double beta = true_residual();
+        double beta = std::sqrt(G.hh[0]);
         int status = MPS_NOT_CONVERGED;
         if (bnorm == 0.0) {
             fill<double>(c, u, g.ng(), 0.0);
@@ -3735,7 +3756,7 @@ int mps_gmres(mps_ctx *c, const double *b, double *x, int m, int max_restarts, d
         // queued, costs an extra preconditioned step per solve, and the
         // coupled solves converge in 1-3 steps.)
         ArnoldiDev A = arnoldi_view(G);
-        double *dh2 = arn_h2(G), *dny = arn_ny(G), *dwn2 = arn_wn2(G);
+        double *dh2 = arn_h2(G), *dny = arn_ny(G);
         const double tolb = tol * bnorm;
         for (int rs = 0; rs < max_restarts && status != MPS_OK; ++rs) {
             if (!std::isfinite(beta)) {
@@ -3751,15 +3772,15 @@ int mps_gmres(mps_ctx *c, const double *b, double *x, int m, int max_restarts, d
             scale_from(c, G.w, G.V[0], A.gv);
             int queued = 0;
             for (int j = 0; j < m; ++j) {
-                precondition(c, G.V[j], G.Z[j]);
-                matvec(c, c->L64, G.Z[j], G.w);
+                const int nv = j + 1;
+                precondition_matvec(c, G, G.V[j], G.Z[j], G.w, G.V.data(), nv, G.dh);
+                if (nv > kDotRegs)
+                    multidot_dev(c, G, G.w, G.V.data() + kDotRegs, nv - kDotRegs, G.dh + kDotRegs);
                 // classical Gram-Schmidt with one re-orthogonalisation pass
-                multidot_dev(c, G, G.w, G.V.data(), j + 1, G.dh);
-                multiaxpy_dev(c, G.w, G.V.data(), j + 1, G.dh, nullptr, nullptr);
-                multidot_dev(c, G, G.w, G.V.data(), j + 1, dh2);
-                multiaxpy_dev(c, G.w, G.V.data(), j + 1, dh2, nullptr, dwn2);
-                hipLaunchKernelGGL(k_arnoldi_step, dim3(1), dim3(64), 0, c->stream, A, j, kArnLd,
-                                   (const double *)G.dh, (const double *)dh2, (const double *)dwn2, tolb);
+                multiaxpy_dots(c, G, G.w, G.V.data(), nv, G.dh, dh2);
+                const int np = multiaxpy_dev(c, G.w, G.V.data(), nv, dh2, nullptr);
+                hipLaunchKernelGGL(k_arnoldi_step, dim3(1), block(), 0, c->stream, A, j, kArnLd, (const double *)G.dh,
+                                   (const double *)dh2, (const double *)c->partials, np, tolb);
                 scale_from(c, G.w, G.V[j + 1], A.hn);
                 HIPCHK(hipMemcpyAsync(G.hflag + j, A.state, sizeof(int), hipMemcpyDeviceToHost, c->stream));
                 HIPCHK(hipEventRecord(G.ev[j], c->stream));
@@ -3768,7 +3789,7 @@ int mps_gmres(mps_ctx *c, const double *b, double *x, int m, int max_restarts, d
                 if (G.hflag[j]) break;
             }
             hipLaunchKernelGGL(k_arnoldi_solve, dim3(1), dim3(64), 0, c->stream, A, kArnLd, dny);
-            multiaxpy_dev(c, u, G.Z.data(), queued, dny, A.state + 1, nullptr);
+            multiaxpy_dev(c, u, G.Z.data(), queued, dny, A.state + 1);
             HIPCHK(hipMemcpyAsync(G.hflag + kMaxVec, A.state, 3 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
             beta = true_residual();
             if (G.hflag[kMaxVec + 2]) {

@@ -289,10 +289,15 @@ __device__ __forceinline__ T gs_update(const Lev<T> &L, T b, T of, T dg)
     return (b - of) / dg;
 }
 
+// a field read as another type
+struct AsDouble {
+    const float *p;
+    __device__ __forceinline__ double operator[](long long c) const { return (double)p[c]; }
+};
+
 // diag and offdiag of cell (i,j,k) at address c for the current u.
-template <typename T, int OP, bool VEL, bool REAC>
-__device__ __forceinline__ void row(const Lev<T> &L, const T *__restrict__ u, int i, int j, int k,
-                                    long long c, T &dg, T &of)
+template <typename T, int OP, bool VEL, bool REAC, typename U>
+__device__ __forceinline__ void row_of(const Lev<T> &L, U u, int i, int j, int k, long long c, T &dg, T &of)
 {
     if (OP != OP_STENCIL && !VEL) {
         const long long sy = L.sy, sz = L.sz;
@@ -354,6 +359,13 @@ __device__ __forceinline__ void row(const Lev<T> &L, const T *__restrict__ u, in
     if (L.timederiv) d = d + T(1) / L.dt;
     dg = d;
     of = o;
+}
+
+template <typename T, int OP, bool VEL, bool REAC>
+__device__ __forceinline__ void row(const Lev<T> &L, const T *__restrict__ u, int i, int j, int k,
+                                    long long c, T &dg, T &of)
+{
+    row_of<T, OP, VEL, REAC, const T *__restrict__>(L, u, i, j, k, c, dg, of);
 }
 
 // The seven row coefficients (centre and the six neighbours) of an
@@ -1271,28 +1283,125 @@ __global__ void __launch_bounds__(kBlock) k_multiaxpy(Lev<double> L, double *w, 
     }
 }
 
-// out = A u over the interior (ghosted output)
-template <typename T, int OP, bool VEL, bool REAC>
-__global__ void __launch_bounds__(kBlock) k_matvec(Lev<T> L, const T *__restrict__ u, T *out)
+// The vectors of one pass whose products are kept in registers; solves that
+// need more steps take the further products from k_multidot.
+constexpr int kDotRegs = 4;
+
+// block partials of the kDotRegs sums d: partials[q * nblocks + block]
+__device__ __forceinline__ void dot_partials(const double *d, int nv, double *partials)
 {
-    int i, j, k;
-    long long c;
-    if (!cell_of(L, i, j, k, c)) return;
-    T dg, of;
-    row<T, OP, VEL, REAC>(L, u, i, j, k, c, dg, of);
-    out[c] = dg * u[c] + of;
+    const int nblocks = gridDim.x * gridDim.y, bid = blockIdx.x + gridDim.x * blockIdx.y;
+#pragma unroll
+    for (int q = 0; q < kDotRegs; ++q) {
+        if (q >= nv) continue;
+        const double s = block_sum(d[q]);
+        if (threadIdx.x == 0) partials[(long long)q * nblocks + bid] = s;
+        __syncthreads();
+    }
+}
+
+// w = A z and its products with the first nv <= kDotRegs vectors. z is u, or,
+// where u is the FP32 cycle's correction, its copy in FP64, which is written.
+// An FP32 solve's step at 129^3 (17 MB fields, SG rows): 37 us, against 7 for
+// the copy, 32 for the product and 8 for one dot product, each its own pass
+// over memory; the whole step of five species went from 7.07 to 6.61 ms with
+// this, k_multiaxpy_dots, the cycle's zero start unread and one read-back
+// for both first norms.
+template <typename U, int OP, bool VEL, bool REAC>
+__global__ void __launch_bounds__(kBlock) k_matvec_dots(Lev<double> L, const U *__restrict__ u, double *z, double *w,
+                                                        VecList V, int nv, double *partials)
+{
+    int i, j;
+    double d[kDotRegs] = {};
+    if (cell_ij(L, i, j)) {
+        for (int k = blockIdx.y + 1; k <= L.nz; k += gridDim.y) {
+            const long long c = (long long)i + (long long)L.sy * j + L.sz * k;
+            double dg, of, uc;
+            if constexpr (sizeof(U) == 4) {
+                const AsDouble a{u};
+                row_of<double, OP, VEL, REAC, AsDouble>(L, a, i, j, k, c, dg, of);
+                uc = a[c];
+                z[c] = uc;
+            } else {
+                row<double, OP, VEL, REAC>(L, u, i, j, k, c, dg, of);
+                uc = u[c];
+            }
+            const double x = dg * uc + of;
+            w[c] = x;
+#pragma unroll
+            for (int q = 0; q < kDotRegs; ++q)
+                if (q < nv) d[q] += x * V.v[q][c];
+        }
+    }
+    dot_partials(d, nv, partials);
+}
+
+// w = w - sum_q h[q] v_q over the interior (q < nv) and the new w's products
+// with the first min(nv, kDotRegs) vectors, which are read once
+__global__ void __launch_bounds__(kBlock) k_multiaxpy_dots(Lev<double> L, double *w, VecList V, const double *h, int nv,
+                                                          double *partials)
+{
+    int i, j;
+    double d[kDotRegs] = {};
+    if (cell_ij(L, i, j)) {
+        for (int k = blockIdx.y + 1; k <= L.nz; k += gridDim.y) {
+            const long long c = (long long)i + (long long)L.sy * j + L.sz * k;
+            double x = w[c], v[kDotRegs];
+#pragma unroll
+            for (int q = 0; q < kDotRegs; ++q) {
+                v[q] = q < nv ? V.v[q][c] : 0.0;
+                if (q < nv) x = x - h[q] * v[q];
+            }
+            for (int q = kDotRegs; q < nv; ++q) x = x - h[q] * V.v[q][c];
+            w[c] = x;
+#pragma unroll
+            for (int q = 0; q < kDotRegs; ++q) d[q] += x * v[q];
+        }
+    }
+    dot_partials(d, min(nv, kDotRegs), partials);
+}
+
+// dst = src with ghosts, and block partials of its square
+__global__ void __launch_bounds__(kBlock) k_interior_in_sq(Lev<double> L, const double *src, double *dst_ghosted,
+                                                           double *partials)
+{
+    int i, j;
+    double sq = 0.0;
+    if (cell_ij(L, i, j)) {
+        for (int k = blockIdx.y + 1; k <= L.nz; k += gridDim.y) {
+            const double x = src[(long long)(i - 1) + (long long)L.nx * ((j - 1) + (long long)L.ny * (k - 1))];
+            dst_ghosted[(long long)i + (long long)L.sy * j + L.sz * k] = x;
+            sq += x * x;
+        }
+    }
+    const double s = block_sum(sq);
+    if (threadIdx.x == 0) partials[blockIdx.x + (long long)gridDim.x * blockIdx.y] = s;
+}
+
+// sums of two sets of partials, one block each
+__global__ void __launch_bounds__(kBlock) k_reduce_pair(const double *p0, int n0, const double *p1, int n1, double *out)
+{
+    const double *p = blockIdx.x ? p1 : p0;
+    const int n = blockIdx.x ? n1 : n0;
+    double s = 0.0;
+    for (int t = threadIdx.x; t < n; t += blockDim.x) s += p[t];
+    s = block_sum(s);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 // v = w / s[0] over the interior (ghosts of v stay zero); nothing when s[0]
-// is not positive (an Arnoldi breakdown or NaN leaves v as it is)
-__global__ void __launch_bounds__(kBlock) k_scale(Lev<double> L, const double *w, double *v, const double *s)
+// is not positive (an Arnoldi breakdown or NaN leaves v as it is); f, if
+// given, takes v in FP32 (the right-hand side of the next FP32 cycle)
+__global__ void __launch_bounds__(kBlock) k_scale(Lev<double> L, const double *w, double *v, const double *s, float *f)
 {
     int i, j, k;
     long long c;
     if (!cell_of(L, i, j, k, c)) return;
     const double d = s[0];
     if (!(d > 0.0)) return;
-    v[c] = w[c] / d;
+    const double x = w[c] / d;
+    v[c] = x;
+    if (f) f[c] = (float)x;
 }
 
 // ------------------------------------------------------------------------
@@ -1317,18 +1426,22 @@ __global__ void k_arnoldi_begin(ArnoldiDev A, const double *beta2)
 }
 
 // Arnoldi step j after both Gram-Schmidt passes: column j of H is h + h2,
-// H(j+1, j) = |w| = sqrt(*wn2); the previous rotations and a new one are
+// H(j+1, j) = |w|; the previous rotations and a new one are
 // applied, and the step marks the restart done when |gv(j+1)| <= tolb or
 // |w| <= 1e-300 (breakdown), or flags a NaN. Nothing once done (steps
-// queued past the end of a restart leave H and gv as they are).
-__global__ void k_arnoldi_step(ArnoldiDev A, int j, int ld, const double *h, const double *h2, const double *wn2,
-                               double tolb)
+// queued past the end of a restart leave H and gv as they are). |w|^2 is the
+// sum of the np block partials wp.
+__global__ void __launch_bounds__(kBlock) k_arnoldi_step(ArnoldiDev A, int j, int ld, const double *h, const double *h2,
+                                                         const double *wp, int np, double tolb)
 {
-    if (threadIdx.x | blockIdx.x) return;
+    double wn2 = 0.0;
+    for (int t = threadIdx.x; t < np; t += blockDim.x) wn2 += wp[t];
+    wn2 = block_sum(wn2);
+    if (threadIdx.x) return;
     if (A.state[0]) return;
     double *Hj = A.H + (long long)ld * j;
     for (int i = 0; i <= j; ++i) Hj[i] = h[i] + h2[i];
-    const double hn = sqrt(wn2[0]);
+    const double hn = sqrt(wn2);
     Hj[j + 1] = hn;
     A.hn[0] = hn;
     if (!isfinite(hn)) {
