@@ -873,7 +873,7 @@ __global__ void __launch_bounds__(kBlock) k_sg_stencil(Lev<double> L, RowArrays 
 // swapping rows and swapping columns back. A pivot of zero (or NaN rows)
 // sets *status = -1 (the inverse is then meaningless).
 // 27 cells 21 us, 64 cells 52 us (98 us with the matrix in LDS, one column
-// per lane), 128 cells 162 us, 210 cells 480 us (2.3 us per pivot; 1024 lanes
+// per lane), 128 cells 162 us, 210 cells 453 us (2.2 us per pivot; 1024 lanes
 // with 49 entries each spill: 1000 us). On the host, with the rows copied
 // there and the inverse back, the 210-cell one held a 6.6 ms species step up
 // for more than 2 ms.
@@ -991,7 +991,7 @@ __global__ void __launch_bounds__(kInvThreads) k_dense_inverse_regs(Lev<double> 
             for (int a = 0; a < A; ++a) {
                 const double f = (tr == pr && a == pa) ? -1.0 : scol[buf][tr + 16 * a];
 #pragma unroll
-                for (int b = 0; b < B; ++b) m[a][b] = m[a][b] - f * rk[b];
+                for (int b = 0; b < B; ++b) m[a][b] = fma(-f, rk[b], m[a][b]);
             }
         }
     }
