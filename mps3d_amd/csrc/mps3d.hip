@@ -3477,10 +3477,12 @@ void ensure_transpose(mps_ctx *c)
             const long long ng = c->geom[l].ng();
             LevelBuf<double> &B = c->LT[l];
             B.u = dalloc<double>(ng);
+            B.u2 = dalloc<double>(ng);   // (for the fused sweeps)
             B.b = dalloc<double>(ng);
             B.r = dalloc<double>(ng);
             if (l > 0) B.uold = dalloc<double>(ng);
             fill<double>(c, B.u, ng, 0.0);
+            fill<double>(c, B.u2, ng, 0.0);
             fill<double>(c, B.b, ng, 0.0);
             fill<double>(c, B.r, ng, 0.0);
             if (B.uold) fill<double>(c, B.uold, ng, 0.0);
@@ -3496,7 +3498,6 @@ void ensure_transpose(mps_ctx *c)
     }
     for (int l = 0; l < c->nlev(); ++l) build_stencil(c, c->LT, l, true);
     c->LT.back().inv = c->opts.hierarchy == MPS_HIER_ALIGNED ? c->dinvT : nullptr;
-    HIPCHK(hipStreamSynchronize(c->stream));
     c->transpose_ready = true;
 }
 
