@@ -1726,14 +1726,15 @@ double measure(const mps_ctx *c, double sumsq, double bnorm2)
     return std::sqrt(sumsq / N);
 }
 
-// squared 2-norm of b into d_scalar
+// squared 2-norm of b's interior into d_scalar
 void b_sumsq(mps_ctx *c, const double *b)
 {
-    // residual of u = 0 against b is b itself: reuse the residual kernel
-    // with a zero solution held in the level-0 residual buffer
-    auto &L = c->L64;
-    fill<double>(c, L[0].r, c->geom[0].ng(), 0.0);
-    residual_sumsq<double>(c, L, L[0].r, b, level_op(c, 0));
+    const dim3 gr = red_grid(c->geom[0]);
+    VecList VL{};
+    VL.v[0] = b;
+    hipLaunchKernelGGL(k_multidot, gr, block(), 0, c->stream, view(c, c->L64, 0), b, VL, 1, c->partials);
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), block(), 0, c->stream, (const double *)c->partials,
+                       (int)(gr.x * gr.y), c->d_scalar);
 }
 
 // One outer step of solve_core: the FP32 V-cycle on the defect, the FP64
@@ -3973,8 +3974,7 @@ int mps_solve_transpose(mps_ctx *c, const double *gsrc, double *lambda, int *ncy
         HIPCHK(hipEventRecord(c->ev0, c->stream));
         double bn2 = 0.0;
         if (c->opts.tol_kind == MPS_TOL_REL_L2) {
-            fill<double>(c, L[0].r, g.ng(), 0.0);
-            residual_sumsq<double>(c, L, L[0].r, L[0].b, OP_STENCIL);
+            b_sumsq(c, L[0].b);
             bn2 = read_scalar(c);
         }
         int it = 0;
