@@ -172,6 +172,7 @@ struct mps_ctx {
     mps_grid grid{};
     mps_opts opts{};
     int device = 0;
+    int cus = 256;                       // compute units of the device
     hipStream_t stream = nullptr;
     hipStream_t stream2 = nullptr;       // the coarsest inverse, beside the set-up
     std::vector<Geom> geom;
@@ -912,8 +913,8 @@ void launch_bottom(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, int op, T *wo
 #ifndef MPS_SWEEP_TY
 #define MPS_SWEEP_TY 8
 #endif
-// (the most planes per z-chunk; k_sweep_fast splits nz into ceil(nz / KZ)
-// even chunks: at 257^3, 15 chunks of 17-18 planes, 3840 blocks, three
+// (the most planes per z-chunk; k_sweep_fast splits nz into even chunks,
+// fast_chunks: at 257^3, 15 chunks of 17-18 planes, 3840 blocks, three
 // rounds of the five blocks per CU that the FP32 sweep's LDS and VGPRs allow)
 #ifndef MPS_SWEEP_KZ
 #define MPS_SWEEP_KZ 18
@@ -932,6 +933,38 @@ GhostD<T> ghost_multipliers(const mps_ctx *c, const Lev<T> &v)
     return G;
 }
 
+// z-chunks of a fast sweep over cols tiles: whole rounds of the blocks that
+// the chip holds of this kernel (by its LDS and registers: 3 a CU for FP64
+// rows from D, 4 for explicit FP64 rows, 5 for FP32), of the rounds the one
+// with the fewest steps in a row. A chunk of kz planes takes kz + 3 steps, and
+// a last round with few blocks takes as long as a full one: at 128^3 in FP64,
+// 26 chunks (1664 blocks, whatever the kernel) took 27.3 and 51.9 us (rows
+// from D; explicit), the 12 and 16 of this rule 20.2 and 46.4; at 161 x 97 x
+// 129 rows from D took 25.8 with 22 chunks, 20.9 with 12. At least 2 planes a chunk, at most
+// kSweepKZ (the tile's lines stay in L2 for the neighbours).
+template <auto Kernel>
+int fast_chunks(const mps_ctx *c, int nz, long long cols)
+{
+    static const int per_cu = [&] {
+        int n = 0;
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)Kernel,
+                                                                         kSweepTX * kSweepTY, 0);
+        return e == hipSuccess && n > 0 ? n : 4;
+    }();
+    const long long held = (long long)per_cu * c->cus;
+    int best = (nz + kSweepKZ - 1) / kSweepKZ;
+    long long steps = 0;
+    for (int r = 1; r <= 8; ++r) {
+        const long long n = std::max(1LL, std::min(held * r / cols, nz / 2LL));
+        const long long kz = (nz + n - 1) / n, t = ((cols * n + held - 1) / held) * (kz + 3);
+        if (kz <= kSweepKZ && (steps == 0 || t < steps)) {
+            best = (int)n;
+            steps = t;
+        }
+    }
+    return best;
+}
+
 // zero_in: sweep from a zero guess, uin unread (fused fast kernels only)
 template <typename T>
 void launch_sweep(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, const T *uin, T *uout, int op, bool zero_in = false)
@@ -940,8 +973,7 @@ void launch_sweep(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, const T *uin, 
     const Geom &g = c->geom[l];
     // (the zero-guess sweeps, which read no u, are not timed)
     KtScope kt(c, l == 0 && !zero_in ? 0 : -2, sizeof(T) == 4);
-// (blocks a z-chunk length aims at: with 1536 the 129^3 level runs 1216
-// blocks, one round of the resident blocks, where 2048 gave 1664)
+// (blocks a z-chunk length of k_sweep and k_sweep_ref aims at)
 #ifndef MPS_SWEEP_TARGET
 #define MPS_SWEEP_TARGET 1536
 #endif
@@ -966,38 +998,33 @@ void launch_sweep(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, const T *uin, 
     // k_sweep_fast: on k TX + 1 columns (rows) k tiles, the last extended
     // by the remaining one
     auto tiles = [](int n, int t) { return (n > t && n % t == 1) ? n / t : (n + t - 1) / t; };
-    const dim3 grf((unsigned)tiles(g.nx, kSweepTX), (unsigned)tiles(g.ny, kSweepTY), gr.z);
+    const int tx = tiles(g.nx, kSweepTX), ty = tiles(g.ny, kSweepTY);
+    auto fast = [&](auto O, auto R) {
+        auto run = [&](auto Z) {
+            constexpr auto kernel = k_sweep_fast<T, decltype(O)::value, decltype(R)::value, kSweepTX, kSweepTY,
+                                                 decltype(Z)::value>;
+            const int n = fast_chunks<kernel>(c, g.nz, (long long)tx * ty);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)tx, (unsigned)ty, (unsigned)n), dim3(kSweepTX * kSweepTY), 0,
+                               c->stream, v, uin, uout, (const T *)L[l].b, (g.nz + n - 1) / n, zg0, zg1);
+        };
+        if (zero_in) run(BoolC<true>{});
+        else run(BoolC<false>{});
+    };
     auto go = [&](auto O, auto R) {
-        if (v.fast && zero_in)
-            hipLaunchKernelGGL(
-                (k_sweep_fast<T, decltype(O)::value, decltype(R)::value, kSweepTX, kSweepTY, true>), grf,
-                dim3(kSweepTX * kSweepTY), 0, c->stream, v, uin, uout, (const T *)L[l].b, kz, zg0, zg1);
-        else if (v.fast)
-            hipLaunchKernelGGL(
-                (k_sweep_fast<T, decltype(O)::value, decltype(R)::value, kSweepTX, kSweepTY, false>), grf,
-                dim3(kSweepTX * kSweepTY), 0, c->stream, v, uin, uout, (const T *)L[l].b, kz, zg0, zg1);
+        if (v.fast)
+            fast(O, R);
         else
             hipLaunchKernelGGL((k_sweep<T, decltype(O)::value, decltype(R)::value, kSweepTX, kSweepTY>), gr,
                                dim3(kSweepTX * kSweepTY), 0, c->stream, v, uin, uout, (const T *)L[l].b, kz);
     };
     if (op == OP_STENCIL && L[l].fc[1]) {
         // the same rows from their face form (conductance coarse levels)
-        if (zero_in)
-            hipLaunchKernelGGL((k_sweep_fast<T, OP_FACES, false, kSweepTX, kSweepTY, true>), grf,
-                               dim3(kSweepTX * kSweepTY), 0, c->stream, v, uin, uout, (const T *)L[l].b, kz, zg0, zg1);
-        else
-            hipLaunchKernelGGL((k_sweep_fast<T, OP_FACES, false, kSweepTX, kSweepTY, false>), grf,
-                               dim3(kSweepTX * kSweepTY), 0, c->stream, v, uin, uout, (const T *)L[l].b, kz, zg0, zg1);
+        fast(IntC<OP_FACES>{}, BoolC<false>{});
     } else if (op == OP_STENCIL) {
         // explicit rows carry their own reaction and time terms; the fast
         // kernel's arithmetic for them is the per-level kernels' in either
         // arithmetic mode
-        if (zero_in)
-            hipLaunchKernelGGL((k_sweep_fast<T, OP_STENCIL, false, kSweepTX, kSweepTY, true>), grf,
-                               dim3(kSweepTX * kSweepTY), 0, c->stream, v, uin, uout, (const T *)L[l].b, kz, zg0, zg1);
-        else
-            hipLaunchKernelGGL((k_sweep_fast<T, OP_STENCIL, false, kSweepTX, kSweepTY, false>), grf,
-                               dim3(kSweepTX * kSweepTY), 0, c->stream, v, uin, uout, (const T *)L[l].b, kz, zg0, zg1);
+        fast(IntC<OP_STENCIL>{}, BoolC<false>{});
     } else if (op == OP_REF) {
         if (c->has_reac) go(IntC<OP_REF>{}, BoolC<true>{});
         else go(IntC<OP_REF>{}, BoolC<false>{});
@@ -2263,6 +2290,7 @@ int mps_create(mps_ctx **out, const mps_grid *grid, const mps_opts *opts)
     }
     try {
         HIPCHK(hipGetDevice(&c->device));
+        HIPCHK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
         HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         {
             const char *ng = std::getenv("MPS3D_NO_GRAPHS");
