@@ -700,7 +700,7 @@ int z_chunk(const Geom &g, int tx, int ty, int target_blocks, int kmax)
 #define MPS_RES_KZ 16
 #endif
 #ifndef MPS_RES_TARGET
-#define MPS_RES_TARGET 4096
+#define MPS_RES_TARGET 1024
 #endif
 constexpr int kResTX = MPS_RES_TX, kResTY = MPS_RES_TY, kResRB = MPS_RES_RB, kResKZ = MPS_RES_KZ;
 
@@ -914,11 +914,13 @@ void launch_bottom(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, int op, T *wo
 #define MPS_SWEEP_TY 8
 #endif
 // (the most planes per z-chunk; k_sweep_fast splits nz into even chunks,
-// fast_chunks: at 257^3, 15 chunks of 17-18 planes, 3840 blocks, three
-// rounds of the five blocks per CU that the FP32 sweep's LDS and VGPRs allow)
+// fast_chunks: at 257^3 in FP32 five of 51-52 planes, 1280 blocks, one round of
+// the five blocks per CU that its LDS and VGPRs allow; 91 us a sweep, 76 from
+// a zero guess, where 15 chunks in three rounds took 94 and 83)
 #ifndef MPS_SWEEP_KZ
-#define MPS_SWEEP_KZ 18
+#define MPS_SWEEP_KZ 54
 #endif
+constexpr int kSweepSlabKZ = 18;         // planes that a chunk can hold at least (fused_ok)
 constexpr int kSweepTX = MPS_SWEEP_TX, kSweepTY = MPS_SWEEP_TY, kSweepKZ = MPS_SWEEP_KZ;
 
 // per-face multipliers of the staged ghost coefficient (k_sweep_ref,
@@ -940,10 +942,10 @@ GhostD<T> ghost_multipliers(const mps_ctx *c, const Lev<T> &v)
 // a last round with few blocks takes as long as a full one: at 128^3 in FP64,
 // 26 chunks (1664 blocks, whatever the kernel) took 27.3 and 51.9 us (rows
 // from D; explicit), the 12 and 16 of this rule 20.2 and 46.4; at 161 x 97 x
-// 129 rows from D took 25.8 with 22 chunks, 20.9 with 12. At least 2 planes a chunk, at most
-// kSweepKZ (the tile's lines stay in L2 for the neighbours).
+// 129 rows from D took 25.8 with 22 chunks, 20.9 with 12. At least 2 planes a chunk, at
+// most kSweepKZ and what a buffer resource spans.
 template <auto Kernel>
-int fast_chunks(const mps_ctx *c, int nz, long long cols)
+int fast_chunks(const mps_ctx *c, int nz, long long cols, long long plane_bytes)
 {
     static const int per_cu = [&] {
         int n = 0;
@@ -952,12 +954,13 @@ int fast_chunks(const mps_ctx *c, int nz, long long cols)
         return e == hipSuccess && n > 0 ? n : 4;
     }();
     const long long held = (long long)per_cu * c->cus;
-    int best = (nz + kSweepKZ - 1) / kSweepKZ;
+    const long long kmax = std::min<long long>(kSweepKZ, ((1LL << 31) - 1) / plane_bytes - 4);
+    int best = (int)((nz + kmax - 1) / kmax);
     long long steps = 0;
     for (int r = 1; r <= 8; ++r) {
         const long long n = std::max(1LL, std::min(held * r / cols, nz / 2LL));
         const long long kz = (nz + n - 1) / n, t = ((cols * n + held - 1) / held) * (kz + 3);
-        if (kz <= kSweepKZ && (steps == 0 || t < steps)) {
+        if (kz <= kmax && (steps == 0 || t < steps)) {
             best = (int)n;
             steps = t;
         }
@@ -977,7 +980,7 @@ void launch_sweep(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, const T *uin, 
 #ifndef MPS_SWEEP_TARGET
 #define MPS_SWEEP_TARGET 1536
 #endif
-    const int kz = z_chunk(g, kSweepTX, kSweepTY, MPS_SWEEP_TARGET, kSweepKZ);
+    const int kz = z_chunk(g, kSweepTX, kSweepTY, MPS_SWEEP_TARGET, kSweepSlabKZ);
     dim3 gr((unsigned)((g.nx + kSweepTX - 1) / kSweepTX), (unsigned)((g.ny + kSweepTY - 1) / kSweepTY),
             (unsigned)((g.nz + kz - 1) / kz));
     if (v.fast && op == OP_REF && !c->has_reac && c->sweep_ref && v.omega == T(1) &&
@@ -1003,7 +1006,7 @@ void launch_sweep(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, const T *uin, 
         auto run = [&](auto Z) {
             constexpr auto kernel = k_sweep_fast<T, decltype(O)::value, decltype(R)::value, kSweepTX, kSweepTY,
                                                  decltype(Z)::value>;
-            const int n = fast_chunks<kernel>(c, g.nz, (long long)tx * ty);
+            const int n = fast_chunks<kernel>(c, g.nz, (long long)tx * ty, (long long)v.sz * (int)sizeof(T));
             hipLaunchKernelGGL(kernel, dim3((unsigned)tx, (unsigned)ty, (unsigned)n), dim3(kSweepTX * kSweepTY), 0,
                                c->stream, v, uin, uout, (const T *)L[l].b, (g.nz + n - 1) / n, zg0, zg1);
         };
@@ -1045,7 +1048,7 @@ bool fused_ok(const mps_ctx *c, const std::vector<LevelBuf<T>> &L, int l, int op
     // needs; rows formed from coefficients are fused only without
     // convection (the fused kernels have no upwind terms)
     const Geom &g = c->geom[l];
-    const long long slab = (long long)(kSweepKZ + 4) * (g.nx + 2) * (g.ny + 2) * (long long)sizeof(T);
+    const long long slab = (long long)(kSweepSlabKZ + 4) * (g.nx + 2) * (g.ny + 2) * (long long)sizeof(T);
     return (op == OP_STENCIL || !c->has_vel) && L[l].u2 && g.ng() < (1LL << 31) && slab < (1LL << 31);
 }
 
