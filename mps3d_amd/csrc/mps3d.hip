@@ -2517,22 +2517,32 @@ int mps_set_bc(mps_ctx *c, const int codes[6], const double *const faces[6])
             c->transpose_ready = false;
             return MPS_OK;
         }
+        // Host faces, or some of each: every copy is on the context's stream,
+        // after the calls queued there, whose ghost values may still be read
+        // from faces0 and whose device faces may still be written. (The
+        // stream is a non-blocking one: a copy on the null stream waits for
+        // none of it.)
+        if (const int st = after_null_stream(c)) return st;
         const int nl = c->nlev();
         c->faces_host.assign((size_t)nl * 6, {});
+        std::vector<std::vector<float>> faces32;
         const Geom &g0 = c->geom[0];
         const long long fsz[6] = {(long long)g0.ny * g0.nz, (long long)g0.ny * g0.nz, (long long)g0.nx * g0.nz,
                                   (long long)g0.nx * g0.nz, (long long)g0.nx * g0.ny, (long long)g0.nx * g0.ny};
         for (int f = 0; f < 6; ++f) {
             auto &h = c->faces_host[f];
             h.assign(fsz[f], 0.0);
-            if (faces && faces[f]) {
-                if (is_device_ptr(faces[f]))
-                    HIPCHK(hipMemcpy(h.data(), faces[f], fsz[f] * sizeof(double), hipMemcpyDeviceToHost));
-                else
-                    std::memcpy(h.data(), faces[f], fsz[f] * sizeof(double));
-            }
+            if (!faces || !faces[f]) continue;
+            if (is_device_ptr(faces[f]))
+                HIPCHK(hipMemcpyAsync(h.data(), faces[f], fsz[f] * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+            else
+                std::memcpy(h.data(), faces[f], fsz[f] * sizeof(double));
+        }
+        HIPCHK(hipStreamSynchronize(c->stream));
+        for (int f = 0; f < 6; ++f) {
             if (!c->faces0[f]) c->faces0[f] = dalloc<double>(fsz[f]);
-            HIPCHK(hipMemcpy(c->faces0[f], h.data(), fsz[f] * sizeof(double), hipMemcpyHostToDevice));
+            HIPCHK(hipMemcpyAsync(c->faces0[f], c->faces_host[f].data(), fsz[f] * sizeof(double),
+                                  hipMemcpyHostToDevice, c->stream));
         }
         // coarse faces: 4-child mean per level (restrict_boundary,
         // mgridsteps.f90:55-128), used by the ghost rule of prolongation1
@@ -2556,16 +2566,20 @@ int mps_set_bc(mps_ctx *c, const int codes[6], const double *const faces[6])
                                         F[(2 * p - 1) + (size_t)fa[f] * (2 * q - 1)]);
                     auto &B64 = c->L64[l];
                     if (!B64.faces[f]) B64.faces[f] = dalloc<double>(C.size());
-                    HIPCHK(hipMemcpy(B64.faces[f], C.data(), C.size() * sizeof(double), hipMemcpyHostToDevice));
+                    HIPCHK(hipMemcpyAsync(B64.faces[f], C.data(), C.size() * sizeof(double), hipMemcpyHostToDevice,
+                                          c->stream));
                     if (c->opts.precision == MPS_PREC_FP32_DC) {
-                        std::vector<float> cf(C.begin(), C.end());
+                        faces32.emplace_back(C.begin(), C.end());
+                        const auto &cf = faces32.back();
                         auto &B32 = c->L32[l];
                         if (!B32.faces[f]) B32.faces[f] = dalloc<float>(cf.size());
-                        HIPCHK(hipMemcpy(B32.faces[f], cf.data(), cf.size() * sizeof(float), hipMemcpyHostToDevice));
+                        HIPCHK(hipMemcpyAsync(B32.faces[f], cf.data(), cf.size() * sizeof(float),
+                                              hipMemcpyHostToDevice, c->stream));
                     }
                 }
             }
         }
+        HIPCHK(hipStreamSynchronize(c->stream));   // (the host copies are done with)
         c->bc_set = true;
         touch_gen(c);
         c->transpose_ready = false;

@@ -154,7 +154,7 @@ class FieldSolver:
     def __exit__(self, *a):
         self.close()
 
-    def order_torch_in(self, faces=False):
+    def order_torch_in(self):
         """Orders the context's stream after torch's current stream (device-
         side, no host wait): tensors torch is still writing are complete
         before the library reads them. Every entry point that takes device
@@ -165,7 +165,7 @@ class FieldSolver:
         if self._ext is None:
             self._ext = torch.cuda.ExternalStream(self.lib.mps_stream(self._h))
         cur = torch.cuda.current_stream()
-        if cur.cuda_stream != 0 or faces:
+        if cur.cuda_stream != 0:
             self._ext.wait_stream(cur)
         self._torch_call = True
 
@@ -190,8 +190,7 @@ class FieldSolver:
             if want is not None and a.numel() != want:
                 raise ValueError("device array has %d elements, expected %d" % (a.numel(), want))
             if not self._torch_call:
-                # (mps_set_bc reads faces of a mixed set with the host's copies)
-                self.order_torch_in(kind == "f")
+                self.order_torch_in()
             return C.c_void_p(a.data_ptr())
         arr = np.asarray(a, dtype=np.float64)
         if kind == "g":
