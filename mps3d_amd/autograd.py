@@ -161,6 +161,25 @@ class Operator:
         self.solver.close()
 
 
+def own_methods(obj, cls, methods):
+    """Whether obj is a cls whose methods (name: function) are cls's own,
+    replaced neither on the object nor on the class."""
+    return type(obj) is cls and methods.keys().isdisjoint(vars(obj)) and \
+        all(vars(cls).get(k) is f for k, f in methods.items())
+
+
+_OPERATOR = {k: vars(Operator)[k] for k in ("configure", "solve", "advance")}
+
+
+def advance(op, rhs, x0, vel=None, scale=1.0):
+    """The interior solution of op for velocities scale * vel, outside
+    autograd: an Operator scales them as it pads them; one of the caller's is
+    called as linear_solve calls it, by configure(vel, rhs) and solve(x0)."""
+    if own_methods(op, Operator, _OPERATOR):
+        return op.advance(rhs, x0, vel, scale)
+    return linear_solve(op, rhs, None if vel is None else tuple(scale * v for v in vel), x0=x0)
+
+
 class LinearSolve(torch.autograd.Function):
     """x = A(v)^-1 b with the hand-written adjoint in backward."""
 

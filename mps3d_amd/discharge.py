@@ -45,7 +45,7 @@ import torch
 from torch.utils.checkpoint import checkpoint
 
 from . import _lib as M
-from .autograd import Operator, linear_solve, native_fields
+from .autograd import Operator, advance, linear_solve, native_fields, own_methods
 
 E_CHARGE = 1.602176634e-19
 EPS0 = 8.8541878128e-12
@@ -238,17 +238,13 @@ class Discharge:
         return torch.cat([q[:1], z, q[-1:]], dim=0)
 
     # ------------------------------------------------------------ one step
-    # the methods whose work the native step does in its own passes
-    _PIECES = frozenset(("potential", "efield", "mean_energy", "rates", "thermal_outflow", "solve_species",
-                         "solve_energy"))
-
     def _native(self, dens, neps, V):
         """The library's description of this step, or None where the step is
         to be built from tensor operations: where a gradient is wanted, a
         method is replaced, a rate is a function of the caller's, or a field
         is not a plain contiguous one of the model's shape on the current
         GPU."""
-        if type(self) is not Discharge or not self._PIECES.isdisjoint(self.__dict__) or self.dev.type != "cuda":
+        if not own_methods(self, Discharge, _PIECES) or self.dev.type != "cuda":
             return None
         ns, nr, nz = len(self.species), len(self.reactions), self.shape[0]
         num = (int, float)
@@ -277,7 +273,7 @@ class Discharge:
                     d.cbar[k] = math.sqrt(8.0 * E_CHARGE * self.Tg_eV / (math.pi * s.mass))
         for r, re in enumerate(self.reactions):
             arr = type(re.rate) is _Arrhenius
-            if type(re) is not Reaction:
+            if not own_methods(re, Reaction, _RATE):
                 return None
             rate, ea = (re.rate.A, re.rate.Ea) if arr else (re.rate, 0.0)
             if not all(isinstance(v, num) for v in (rate, ea, re.energy)) or len(re.reactants) > M.DIS_ORDER:
@@ -316,12 +312,12 @@ class Discharge:
         out = []
         for k, (s, nsp) in enumerate(zip(self.species, dens)):
             drift = s.charge != 0 and s.mu > 0
-            out.append(self.ops[k].advance(rhs[k], nsp, tuple(E) if drift else None,
-                                           math.copysign(s.mu, s.charge) if drift else 1.0))
+            out.append(advance(self.ops[k], rhs[k], nsp, tuple(E) if drift else None,
+                               math.copysign(s.mu, s.charge) if drift else 1.0))
         if not self.energy:
             return tuple(out), None
         ve = -(5.0 / 3.0) * self.species[d.electron].mu
-        return tuple(out), self.energy_op.advance(rhs[-1], neps, tuple(E), ve)
+        return tuple(out), advance(self.energy_op, rhs[-1], neps, tuple(E), ve)
 
     def step(self, dens, neps, V):
         """dens: tuple of species densities; neps: electron energy density
@@ -424,6 +420,12 @@ class Discharge:
             op.close()
         if self.energy:
             self.energy_op.close()
+
+
+# the methods whose work the native step does in its own passes
+_PIECES = {k: vars(Discharge)[k] for k in ("potential", "efield", "mean_energy", "rates", "thermal_outflow",
+                                           "solve_species", "solve_energy")}
+_RATE = {"coefficient": Reaction.coefficient}
 
 
 # ------------------------------------------------------------------ workloads

@@ -5,7 +5,8 @@ passes do the same operations in the same order without contraction, so the
 bar is 1e-14 relative to the largest value (exp may differ by an ulp), and
 bitwise for the padded fields. Where a step may not take the passes it does
 not: gradients wanted, replaced methods, rates of the caller's, other
-layouts."""
+layouts. Operators of the caller's are called as they are where a step is
+built from tensor operations."""
 import pytest
 import torch
 
@@ -121,4 +122,69 @@ def test_steps_that_stay_tensor_operations(gpu):
     del m.solve_species
     m.reactions[0].rate = lambda eps: 1e-13 * torch.exp(-15.0 / eps)
     assert m._native(dens, neps, V) is None
+    m.close()
+
+
+def recorder(seen, factor):
+    """configure and solve as LinearSolve calls them, with nothing else."""
+    def configure(self, vel=None, rhs=None):
+        seen.append([rhs.clone()] + [v.clone() for v in vel or ()])
+        self.given = rhs
+
+    def solve(self, x0=None):
+        return AG.pad(factor * self.given)
+
+    return configure, solve
+
+
+@pytest.mark.parametrize("how", ["object", "subclass", "instance", "class"])
+@pytest.mark.parametrize("form", ["energy", "local"])
+def test_operators_of_the_callers(gpu, how, form, monkeypatch):
+    n, out = 8, []
+    V = torch.tensor([800.0, -300.0], dtype=F64, device="cuda")
+    for cls in (DS.Discharge, Torch):
+        m = build(cls, form, n)
+        seen = []
+        configure, solve = recorder(seen, 0.9 * m.dt)
+        body = {"configure": configure, "solve": solve}
+        ops = m.ops + ([m.energy_op] if m.energy else [])
+        if how == "object":
+            m.ops = [type("Op", (), body)() for _ in m.ops]
+            if m.energy:
+                m.energy_op = type("Op", (), body)()
+        with monkeypatch.context() as mp:
+            for op in ops:
+                if how == "subclass":
+                    op.__class__ = type("Op", (AG.Operator,), body)
+                elif how == "instance":
+                    op.configure, op.solve = configure.__get__(op), solve.__get__(op)
+            if how == "class":
+                for k, f in body.items():
+                    mp.setattr(AG.Operator, k, f)
+                m.poisson.__class__ = type("Op", (AG.Operator,), dict(body, solve=recorder(seen, 1e-9 * m.h ** 2)[1]))
+            dens, neps = state(m, n)
+            m.step(dens, neps, V)
+        out.append(seen)
+        for op in ops + [m.poisson]:
+            op.close()
+    assert len(out[0]) == len(out[1]) == len(ops) + (how == "class")
+    # (where the potential is not replaced the velocities hold a solve to 1e-10)
+    bar = 1e-14 if how == "class" else 1e-8
+    for a, b in zip(*out):
+        assert len(a) == len(b)
+        for x, y in zip(a, b):
+            assert float((x - y).abs().max()) <= bar * float(y.abs().max())
+
+
+def test_methods_replaced_on_the_class(gpu, monkeypatch):
+    m = build(DS.Discharge, "energy", 6)
+    dens, neps = state(m, 6)
+    V = torch.tensor([800.0], dtype=F64, device="cuda")
+    for cls, name in [(DS.Discharge, k) for k in ("potential", "efield", "mean_energy", "rates", "thermal_outflow",
+                                                  "solve_species", "solve_energy")] + [(DS.Reaction, "coefficient")]:
+        with monkeypatch.context() as mp:
+            old = getattr(cls, name)
+            mp.setattr(cls, name, lambda *a, _f=old: _f(*a))
+            assert m._native(dens, neps, V) is None, name
+        assert m._native(dens, neps, V) is not None
     m.close()
