@@ -257,7 +257,9 @@ class Discharge:
             return None
         d = M.Discharge()
         d.nspecies, d.nreactions, d.energy, d.electron = ns, nr, int(self.energy), -1
-        scalars = [self.dt, self.h, self.Ng, self.Tg_eV, *self.eps_lfa]
+        # (with an energy equation nothing reads the local field's constants)
+        eps0, eps_ref = (0.0, 1.0) if self.energy else self.eps_lfa
+        scalars = [self.dt, self.h, self.Ng, self.Tg_eV, eps0, eps_ref]
         for k, s in enumerate(self.species):
             scalars += [s.charge, s.mu, s.mass]
             if s.name != self.names[k] or not all(isinstance(v, num) for v in scalars):
@@ -291,7 +293,7 @@ class Discharge:
                                                                                      hi.requires_grad):
             return None
         d.rho_coef, d.wall_weight = E_CHARGE / EPS0, 2.0 / (self.h * self.h)
-        d.dt, d.h, d.gas, d.T_gas, (d.eps0, d.eps_ref) = self.dt, self.h, self.Ng, self.Tg_eV, self.eps_lfa
+        d.dt, d.h, d.gas, d.T_gas, d.eps0, d.eps_ref = self.dt, self.h, self.Ng, self.Tg_eV, eps0, eps_ref
         if self.energy:
             e = self.species[d.electron]
             d.neps, d.mu_e = neps.data_ptr(), e.mu

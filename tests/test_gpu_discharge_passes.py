@@ -188,3 +188,16 @@ def test_methods_replaced_on_the_class(gpu, monkeypatch):
             assert m._native(dens, neps, V) is None, name
         assert m._native(dens, neps, V) is not None
     m.close()
+
+
+def test_the_local_field_constants_are_read_where_they_are_used(gpu):
+    # with the energy equation the mean energy takes none of them
+    out = []
+    for lfa in ((1.0, 5e4), None):
+        m = build(DS.Discharge, "energy", 8)
+        m.eps_lfa = lfa
+        dens, neps = state(m, 8)
+        out.append(m.step(dens, neps, torch.tensor([800.0], dtype=F64, device="cuda")))
+        m.close()
+    (a, ea), (b, eb) = out
+    assert all(torch.equal(x, y) for x, y in zip(a + (ea,), b + (eb,)))
