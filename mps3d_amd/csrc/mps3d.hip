@@ -1983,7 +1983,8 @@ int solve_core(mps_ctx *c, double *u, double *b, bool homog, double *history, do
 // global memory, on the aligned hierarchy host_bottom_inverse.
 // The aligned hierarchy refuses a singular coarsest operator: the kernel's
 // verdict is copied to pinned memory behind an event, which
-// finish_bottom_inverse waits for while the finer levels' set-up runs.
+// finish_bottom_inverse waits for while the finer levels' set-up runs. Where
+// the kernel cannot tell, the host's elimination decides.
 int bottom_rows(mps_ctx *c, RowArrays &S)
 {
     const int lb = c->nlev() - 1;
@@ -2015,7 +2016,7 @@ void launch_bottom_inverse(mps_ctx *c)
         if (aligned) throw HipError{hipErrorInvalidValue, "coarsest grid too large for a dense solve"};
         return;   // the reference GMRES stays
     }
-    if (aligned && n > kInvRegsN) return;   // host_bottom_inverse
+    if (aligned && n > kInvRegsN) return;   // (formed on the host)
     const size_t full = (size_t)kBottomMaxDense * kBottomMaxDense;
     if (!c->dinv) c->dinv = dalloc<double>(full);
     if (aligned && !c->dinvT) c->dinvT = dalloc<double>(full);
@@ -2058,25 +2059,14 @@ void launch_bottom_inverse(mps_ctx *c)
     if (!c->L32.empty()) c->L32[lb].inv = c->dinv;
 }
 
-void finish_bottom_inverse(mps_ctx *c)
-{
-    if (!c->inv_pending) return;
-    c->inv_pending = false;
-    HIPCHK(hipEventSynchronize(c->ev_inv));
-    int st;
-    std::memcpy(&st, c->h_scalar + 2, sizeof(int));
-    if (st == 0) return;
-    for (auto &B : c->L64) B.inv = nullptr;
-    for (auto &B : c->L32) B.inv = nullptr;
-    throw HipError{hipErrorInvalidValue, "singular coarsest-level operator"};
-}
-
+// the inverse formed on the host, for the aligned hierarchy's coarsest grids
+// above kInvRegsN cells, and where k_dense_inverse_regs met a pivot too small
+// to tell: throws if a pivot is zero
 void host_bottom_inverse(mps_ctx *c)
 {
     const int lb = c->nlev() - 1;
     const Geom &g = c->geom[lb];
     const int n = (int)g.n();
-    if (!c->mg_ok || c->opts.hierarchy != MPS_HIER_ALIGNED || n <= kInvRegsN) return;
     const long long ng = g.ng();
     std::vector<std::vector<double>> st(ST_N, std::vector<double>(ng, 0.0));
     RowArrays S{};
@@ -2132,10 +2122,28 @@ void host_bottom_inverse(mps_ctx *c)
         for (int q = 0; q < n; ++q) IT[(size_t)q * n + r] = I[(size_t)r * n + q];
     if (!c->dinv) c->dinv = dalloc<double>((size_t)kBottomMaxDense * kBottomMaxDense);
     if (!c->dinvT) c->dinvT = dalloc<double>((size_t)kBottomMaxDense * kBottomMaxDense);
-    HIPCHK(hipMemcpy(c->dinv, I.data(), (size_t)n * n * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->dinvT, IT.data(), (size_t)n * n * sizeof(double), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpyAsync(c->dinv, I.data(), (size_t)n * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->dinvT, IT.data(), (size_t)n * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
     c->L64[lb].inv = c->dinv;
     if (!c->L32.empty()) c->L32[lb].inv = c->dinv;
+}
+
+// the end of a set-up's inverse: waits for the kernel's verdict
+void finish_bottom_inverse(mps_ctx *c)
+{
+    if (c->inv_pending) {
+        c->inv_pending = false;
+        HIPCHK(hipEventSynchronize(c->ev_inv));
+        int st;
+        std::memcpy(&st, c->h_scalar + 2, sizeof(int));
+        if (st == 0) return;
+    } else if (!c->mg_ok || c->opts.hierarchy != MPS_HIER_ALIGNED) {
+        return;
+    }
+    for (auto &B : c->L64) B.inv = nullptr;
+    for (auto &B : c->L32) B.inv = nullptr;
+    host_bottom_inverse(c);
 }
 
 void free_gmres(GmresBufs &G);
@@ -2662,7 +2670,6 @@ int mps_set_coeffs(mps_ctx *c, const double *dcoeff, const double *velx, const d
         launch_bottom_inverse(c);
         for (int l = lb - 1; l >= 0 && rows; --l) build_stencil(c, L, l, false);
         if (c->opts.precision == MPS_PREC_FP32_DC) build_fp32(c);
-        host_bottom_inverse(c);
         HIPCHK(hipGetLastError());
         finish_bottom_inverse(c);
         // host arrays were staged: complete before the call returns; device

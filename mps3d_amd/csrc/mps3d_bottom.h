@@ -870,8 +870,10 @@ __global__ void __launch_bounds__(kBlock) k_sg_stencil(Lev<double> L, RowArrays 
 // by 255 - row, so near-ties go to the lowest row) in cross-lane moves of
 // the vector unit. Rows stay where they are; which row took step kk is
 // recorded and undone in the final scatter, which moves the same values as
-// swapping rows and swapping columns back. A pivot of zero (or NaN rows)
-// sets *status = -1 (the inverse is then meaningless).
+// swapping rows and swapping columns back. A pivot below kPivotFloor of its
+// column's largest entry (or a NaN) sets *status = -1: whether such an
+// operator is singular depends on how its elimination rounds, and the caller
+// leaves the answer, and the inverse, to host_bottom_inverse.
 // 27 cells 21 us, 64 cells 52 us (98 us with the matrix in LDS, one column
 // per lane), 128 cells 162 us, 210 cells 453 us (2.2 us per pivot; 1024 lanes
 // with 49 entries each spill: 1000 us). On the host, with the rows copied
@@ -880,6 +882,11 @@ __global__ void __launch_bounds__(kBlock) k_sg_stencil(Lev<double> L, RowArrays 
 // ------------------------------------------------------------------------
 constexpr int kInvRegsN = 224;
 constexpr int kInvThreads = 512;
+// An elimination with partial pivoting ends in an exact zero only where it
+// leaves rounding errors of the column, some n eps of its largest entry: no-
+// flux operators of 2 to 224 cells end at 5e-14 of it at most, in this
+// kernel's fused arithmetic too; one plane of DIRC faces keeps them above 0.05.
+constexpr double kPivotFloor = 1.0 / (1 << 30);
 constexpr int kDenseThreads = 1024;
 
 // max over the wave of a key >= 0, in lane 63 (row shifts within 16 lanes,
@@ -899,6 +906,7 @@ __global__ void __launch_bounds__(kInvThreads) k_dense_inverse_regs(Lev<double> 
 {
     constexpr int N = 32 * E, A = 2 * E, B = E;
     __shared__ double scol[2][N], srow[2][N];
+    __shared__ double floor_of[N];   // the least pivot of a column that counts as one
     __shared__ int perm[N], pos[N];
     const int nx = L.nx, ny = L.ny, n = L.nx * L.ny * L.nz;
     const int tid = threadIdx.x, tr = tid >> 5, tc = tid & 31, lane = tid & 63;
@@ -923,6 +931,19 @@ __global__ void __launch_bounds__(kInvThreads) k_dense_inverse_regs(Lev<double> 
             }
             m[a][b] = v;
         }
+    }
+    if (tid < n) {
+        // column tid: its diagonal, and its neighbours' entries for this cell
+        const int i = tid % nx + 1, j = (tid / nx) % ny + 1, k = tid / (nx * ny) + 1;
+        const long long c = (long long)i + (long long)L.sy * j + L.sz * k;
+        double v = fabs(S.st[ST_C][c]);
+        if (i > 1) v = fmax(v, fabs(S.st[ST_XP][c - 1]));
+        if (i < nx) v = fmax(v, fabs(S.st[ST_XM][c + 1]));
+        if (j > 1) v = fmax(v, fabs(S.st[ST_YP][c - L.sy]));
+        if (j < ny) v = fmax(v, fabs(S.st[ST_YM][c + L.sy]));
+        if (k > 1) v = fmax(v, fabs(S.st[ST_ZP][c - L.sz]));
+        if (k < L.nz) v = fmax(v, fabs(S.st[ST_ZM][c + L.sz]));
+        floor_of[tid] = kPivotFloor * v;
     }
     unsigned used = 0;   // bit t: row lane + 64 t has been a pivot row
     bool bad = false;
@@ -960,9 +981,9 @@ __global__ void __launch_bounds__(kInvThreads) k_dense_inverse_regs(Lev<double> 
             const unsigned khi = __builtin_amdgcn_readlane((int)(key >> 32), 63);
             // (an unused row below n always exists, so p < n)
             const int p = 255 - (int)(klo & 0xffu);
-            if (khi == 0 && (klo >> 8) == 0) bad = true;
             if ((p & 63) == lane) used |= 1u << (p >> 6);
             const double piv = scol[buf][p];
+            if (!(fabs(piv) > floor_of[kk])) bad = true;
             const int pr = p & 15, pa = p >> 4;
             if (tr == pr) {
 #pragma unroll

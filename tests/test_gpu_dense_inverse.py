@@ -4,7 +4,9 @@ x = A^-1 b, compared with numpy's dense solve of the matrix that find_AX
 gives. Bar: 8 n eps cond(A) relative, the forward error of an inverse formed
 by elimination with partial pivoting and applied by one product, with a
 factor for its constants. Sizes: one cell, the edges of each register
-layout, and above the largest."""
+layout, and above the largest. A singular operator is refused where an
+elimination in FP64, operation by operation, meets a zero pivot, and accepted
+where its rounding leaves one that is not zero."""
 import numpy as np
 import pytest
 
@@ -57,3 +59,52 @@ def test_a_singular_coarsest_operator_is_refused(gpu, n):
         s.set_bc(("ZGRD",) * 6)
         with pytest.raises(M.MpsError, match="singular"):
             s.set_coeffs(np.zeros(n))
+
+
+def eliminates(A):
+    """Whether Gauss-Jordan elimination with partial pivoting meets no zero pivot."""
+    A = A.copy()
+    for c in range(len(A)):
+        p = c + int(np.argmax(np.abs(A[c:, c])))
+        if not abs(A[p, c]) > 0.0:
+            return False
+        A[[c, p]] = A[[p, c]]
+        A[c] *= 1.0 / A[c, c]
+        for r in np.nonzero(A[:, c])[0]:
+            if r != c:
+                A[r] -= A[r, c] * A[c]
+    return True
+
+
+def no_flux_rows(n, length):
+    """The operator with D = 1 and no flux through any face, as find_AX sums it."""
+    N = int(np.prod(n))
+    A = np.zeros((N, N))
+    for r, p in enumerate(np.ndindex(n[::-1])):
+        for d in (2, 1, 0):
+            w = (0.5 * (1.0 + 1.0)) / (length / n[2 - d]) * (1.0 / (length / n[2 - d]))
+            for s in (-1, 1):
+                if 0 <= p[d] + s < n[2 - d]:
+                    A[r, r + s * int(np.prod(n[:2 - d]))] = -w
+                    A[r, r] += w
+    return A
+
+
+def test_a_singular_operator_is_judged_by_its_rounding(gpu):
+    wrong, refused = [], 0
+    for n in ((i, j, k) for i in range(1, 7) for j in range(1, 7) for k in range(1, 7)):
+        # (grids that are their own coarsest level)
+        if np.prod(n) > 100 or min(n) > 3 and all(v % 2 for v in n):
+            continue
+        want = eliminates(no_flux_rows(n, 0.02))
+        refused += not want
+        with FieldSolver(n, (0.02,) * 3, hierarchy="aligned", arith="fast") as s:
+            s.set_bc(("ZGRD",) * 6)
+            try:
+                s.set_coeffs(np.ones(n))
+                got = True
+            except M.MpsError as e:
+                got = "singular" not in str(e)
+        if got != want:
+            wrong.append(n)
+    assert refused > 0 and wrong == []
