@@ -1989,8 +1989,9 @@ int bottom_rows(mps_ctx *c, RowArrays &S)
 {
     const int lb = c->nlev() - 1;
     const Geom &g = c->geom[lb];
-    const bool aligned = c->opts.hierarchy == MPS_HIER_ALIGNED;
-    if (aligned && level_op(c, c->L64, lb) == OP_STENCIL) {
+    // (explicit rows are formed before this on either hierarchy; rows built
+    // from D here would leave their drift and reaction out)
+    if (level_op(c, c->L64, lb) == OP_STENCIL) {
         for (int q = 0; q < ST_N; ++q) S.st[q] = c->L64[lb].st[q];
         return lb;
     }

@@ -6,7 +6,9 @@ by elimination with partial pivoting and applied by one product, with a
 factor for its constants. Sizes: one cell, the edges of each register
 layout, and above the largest. A singular operator is refused where an
 elimination in FP64, operation by operation, meets a zero pivot, and accepted
-where its rounding leaves one that is not zero."""
+where its rounding leaves one that is not zero. On the reference hierarchy
+with Scharfetter-Gummel rows the inverse is of those rows, with their drift
+and reaction."""
 import numpy as np
 import pytest
 
@@ -108,3 +110,27 @@ def test_a_singular_operator_is_judged_by_its_rounding(gpu):
         if got != want:
             wrong.append(n)
     assert refused > 0 and wrong == []
+
+
+@pytest.mark.parametrize("n,p", [((16, 16, 16), (1, 1, 1)), ((24, 24, 24), (3, 3, 3)), ((16, 16, 16), (4, 4, 4)),
+                                 ((56, 56, 40), (7, 7, 5))])
+@pytest.mark.parametrize("prec", ["fp64", "fp32dc"])
+@pytest.mark.parametrize("timederiv", [False, True])
+def test_reference_hierarchy_with_drift_in_fast_arithmetic(gpu, n, p, prec, timederiv):
+    # coarsest grids of 1, 27, 64 and 245 cells; the cycle in exact arithmetic, whose
+    # coarse solve is GMRES, sets the count (one more is allowed)
+    drift = [np.full(n, v, order="F") for v in (1e4, -2e4, 3e4)]
+    reac = np.full(n, -1e6, order="F")
+    b = np.asfortranarray(np.random.default_rng(3).standard_normal(n))
+    count = {}
+    for arith in ("exact", "fast"):
+        with FieldSolver(n, (0.02,) * 3, p=p, hierarchy="ref", flux="sg", arith=arith, precision=prec, tol=1e-10,
+                         tol_kind="rel", max_cycles=30) as s:
+            s.set_bc(("ZGRD",) * 4 + ("DIRC",) * 2, (0.0,) * 4 + (1.0, 2.0))
+            s.set_coeffs(np.full(n, 100.0, order="F"), *drift, reac, b, timederiv, 1e-7)
+            x, y = ghosted(np.zeros(n)), ghosted(np.zeros(n))
+            k, _, _, st = s.solve(x)
+            g, _, gst = s.gmres(b, y, m=30, restarts=1, tol=1e-10)
+            assert st == 0 and gst == 0, (arith, k, g)
+            count[arith] = k, g
+    assert all(f <= e + 1 for f, e in zip(count["fast"], count["exact"])), count
