@@ -225,9 +225,14 @@ class PlasmaRun:
         return {"left": 0, "right": 0, "bottom": 1, "top": 1, "back": 2, "front": 2}[f]
 
     # ------------------------------------------------------------ one step
+    @staticmethod
+    def _dense(faces):
+        """The faces as set_bc takes them."""
+        return [x.contiguous() for x in faces]
+
     def _solve(self, s, u, codes, faces, co, timederiv, dt_s, faces_changed=True, coeffs_changed=True):
         if faces_changed:
-            s.set_bc(codes, [x.contiguous() for x in faces])
+            s.set_bc(codes, faces)
         if coeffs_changed:
             V = co["vel"].view(3, -1)
             s.set_coeffs(co["dcoeff"], V[0], V[1], V[2], co["reac"], co["source"], timederiv, dt_s)
@@ -244,23 +249,27 @@ class PlasmaRun:
         cyc = []
         # Each equation is one row of calls on its context: the transport's
         # coefficients go into arrays kept for the context, and torch works
-        # between the rows only.
+        # between the rows only: faces and densities that are not contiguous
+        # are copied before the row (in it, nothing would order the copy
+        # before the calls that read it).
         # poisson_solve (poissoneq.f90:387-470); the potential's faces stay
         # (poisson_update_bcs changes only 'DZGD' electrodes)
         ions = self.numden[self.ions[0]:self.ions[-1] + 1].reshape(-1)
+        plates = self._dense(self.faces["pot"])
         with self.pois.chained():
             co = self.pois.poisson_transport(self.numden[e].reshape(-1), ions, self.scal["pot"], timederiv=False,
                                              dt=dt_s, out=self._out["pois"])
             # (its coefficients never change: the permittivity-free operator
             # dcoeff = tscale/lscale^2 of poisson_update_transport; only the source)
-            cyc.append(self._solve(self.pois, self.phi_s, self.codes["pot"], self.faces["pot"], co, False, dt_s,
+            cyc.append(self._solve(self.pois, self.phi_s, self.codes["pot"], plates, co, False, dt_s,
                                    faces_changed=self.steps == 0, coeffs_changed=self.steps == 0))
             # update_efield (poissoneq.f90:565-680)
             self.pois.efield(self.phi_s, self.potscale / self.L0, False, out=self.E)
         self.pot = self.phi_s * self.potscale
         # eenergy_solve (eenergyeq.f90:776-840) and update_electrontemp
+        dens = self.numden.reshape(-1)
         with self.ener.chained():
-            co = self.ener.eenergy_transport(self.E.reshape(-1), self.Te.reshape(-1), self.numden.reshape(-1),
+            co = self.ener.eenergy_transport(self.E.reshape(-1), self.Te.reshape(-1), dens,
                                              self.scal["ener"], lscale=self.L0, soln=self.eps_s.reshape(-1),
                                              dt=dt_s, Tg=self.Tg, Pg=self.Pg, out=self._out["ener"])
             self._eenergy_bcs()
@@ -268,9 +277,10 @@ class PlasmaRun:
             self.ener.electron_temp(self.eps_s, self.numden[e], self.eescale, self.etempmin, self.Te)
         self.eps = self.eps_s * self.eescale
         # eden_solve (edeneq.f90:446-523)
+        dens = self.numden.reshape(-1)
         with self.elec.chained():
             co = self.elec.species_transport(ch.especnum, self.E.reshape(-1), self.Te.reshape(-1),
-                                             self.numden.reshape(-1), self.scal["eden"], soln=self.ne_s.reshape(-1),
+                                             dens, self.scal["eden"], soln=self.ne_s.reshape(-1),
                                              dt=dt_s, Tg=self.Tg, Pg=self.Pg,
                                              out=dict(self._out["elec"], prod=self.eprod.view(-1)))
             self._eden_bcs()
@@ -280,22 +290,23 @@ class PlasmaRun:
         # ions_solve (ionseq.f90:560-629): every ion from the same densities,
         # which take the new ion densities after the last one
         for q, sp in enumerate(self.ions):
-            flux = self._ion_faces(q)
+            dens, flux = self.numden.reshape(-1), self._ion_faces(q)
+            faces = self._dense(self.faces["ion"][q])
             with self.ion.chained():
                 co = self.ion.species_transport(sp + 1, self.E.reshape(-1), self.Te.reshape(-1),
-                                                self.numden.reshape(-1), self.scal["ion"],
+                                                dens, self.scal["ion"],
                                                 soln=self.ni_s[q].reshape(-1), dt=dt_s, Tg=self.Tg, Pg=self.Pg,
                                                 out=self._out["ion"])
-                self._ion_bcs(q, sp, flux)
-                cyc.append(self._solve(self.ion, self.ni_s[q], self.codes["spec"], self.faces["ion"][q], co, True,
-                                       dt_s))
+                self._ion_bcs(q, sp, dens, flux)
+                cyc.append(self._solve(self.ion, self.ni_s[q], self.codes["spec"], faces, co, True, dt_s))
         for q, sp in enumerate(self.ions):
             self.numden[sp].copy_(self.ni_s[q] * self.iscale)
         # neutrals_solve (neutralseq.f90:438-508), after it the same update
         for q, sp in enumerate(self.neutrals):
+            dens = self.numden.reshape(-1)
             with self.neut.chained():
                 co = self.neut.species_transport(sp + 1, self.E.reshape(-1), self.Te.reshape(-1),
-                                                 self.numden.reshape(-1), self.scal["neut"],
+                                                 dens, self.scal["neut"],
                                                  soln=self.nn_s[q].reshape(-1), dt=dt_s, Tg=self.Tg, Pg=self.Pg,
                                                  out=dict(self._out["neut"], prod=self.nprod[q].view(-1)))
                 # neutrals_update_transport leaves vel at zero
@@ -342,13 +353,13 @@ class PlasmaRun:
                 flux[k] = faces[k]    # rewritten in place: mps_set_bc copies the faces
         return flux
 
-    def _ion_bcs(self, q, sp, flux):
+    def _ion_bcs(self, q, sp, dens, flux):
         """ions_update_bcs (ionseq.f90:206-476) for ion sp: FLUX faces carry
         the drift outflow mu n E_normal where it leaves the domain, else
         zero."""
         if any(t is not None for t in flux):
             # all FLUX faces of this ion in one launch (mps_ion_drift_faces)
-            self.ion.ion_drift_faces(sp + 1, self.E.reshape(-1), self.numden.reshape(-1),
+            self.ion.ion_drift_faces(sp + 1, self.E.reshape(-1), dens,
                                      self.ni_s[q].reshape(-1), self.vel_scaling, flux)
 
     def _neutral_bcs(self, q, sp):

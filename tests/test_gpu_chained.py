@@ -125,3 +125,41 @@ def test_a_face_written_in_the_row_reaches_a_mixed_set(gpu, hierarchy, precision
     assert float(out[0][0].abs().min()) > 0.0
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("chem", ["ion_elec", "h2_o2"])
+def test_a_plasma_step_launches_nothing_of_torchs_in_its_rows(gpu, chem):
+    # nothing but views, also where faces and densities are strided; and the
+    # same fields as from contiguous ones
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from mps3d_amd import chemistry, plasma
+    deck, make = {"ion_elec": (plasma.ION_ELEC_DECK, chemistry.ion_elec),
+                  "h2_o2": (plasma.H2_O2_DECK, chemistry.h2_o2)}[chem]
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if any(s is not None and s._chained for s in contexts) and not func.is_view:
+                seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    out, seen = [], []
+    for strided in (False, True):
+        run = plasma.PlasmaRun(dict(deck, n=(16, 16, 16), p=(2, 2, 1)), make())
+        contexts = [run.pois, run.ener, run.elec, run.ion, run.neut]
+        if strided:
+            for faces in [run.faces["pot"]] + run.faces["ion"]:
+                for k in range(6):
+                    if not (faces is not run.faces["pot"] and run.codes["spec"][k] == "FLUX"):
+                        faces[k] = faces[k].t().contiguous().t()
+            wide = torch.zeros((2 * run.numden.shape[0],) + run.numden.shape[1:], dtype=F64, device="cuda")
+            wide[::2] = run.numden
+            run.numden = wide[::2]
+        with Watch():
+            for _ in range(2):
+                run.step()
+        out.append([run.numden.clone(), run.phi_s.clone(), run.E.clone(), run.Te.clone(), run.eps_s.clone()])
+        run.close()
+    assert seen == []
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
