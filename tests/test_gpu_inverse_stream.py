@@ -31,3 +31,13 @@ def test_back_to_back_setups(gpu, n, prec):
                 s.solve(x)
                 out.append(x.clone())
     assert all(torch.equal(a, b) for a, b in zip(out[:6], out[6:]))
+
+
+@pytest.mark.parametrize("n,cells", [((25, 25, 25), 64), ((33, 17, 41), 90), ((33, 17, 65), 135), ((49, 33, 25), 140)])
+@pytest.mark.parametrize("prec", ["fp64", "fp32dc"])
+def test_coarsest_grids_of(gpu, n, cells, prec):
+    c = n
+    while min(c) > 3 and all(v % 2 for v in c):
+        c = tuple((v + 1) // 2 for v in c)
+    assert c[0] * c[1] * c[2] == cells
+    test_back_to_back_setups(gpu, n, prec)
