@@ -699,6 +699,11 @@ int z_chunk(const Geom &g, int tx, int ty, int target_blocks, int kmax)
 #ifndef MPS_RES_KZ
 #define MPS_RES_KZ 16
 #endif
+// (blocks the z-chunks of k_residual_planes aim at. 4096 of them overlap better
+// in the kernel itself where a level is long, 39 us for 46 at 129 x 129 x 257
+// in FP64, but one workgroup then sums four times the partials: of solves on
+// twelve grids from 65^3 to 385 x 129 x 129 in both precisions none is more
+// than 1 % faster with 1536, 2048, 3072 or 4096, and several are 2 % slower)
 #ifndef MPS_RES_TARGET
 #define MPS_RES_TARGET 1024
 #endif
@@ -913,15 +918,8 @@ void launch_bottom(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, int op, T *wo
 #ifndef MPS_SWEEP_TY
 #define MPS_SWEEP_TY 8
 #endif
-// (the most planes per z-chunk; k_sweep_fast splits nz into even chunks,
-// fast_chunks: at 257^3 in FP32 five of 51-52 planes, 1280 blocks, one round of
-// the five blocks per CU that its LDS and VGPRs allow; 91 us a sweep, 76 from
-// a zero guess, where 15 chunks in three rounds took 94 and 83)
-#ifndef MPS_SWEEP_KZ
-#define MPS_SWEEP_KZ 54
-#endif
 constexpr int kSweepSlabKZ = 18;         // planes that a chunk can hold at least (fused_ok)
-constexpr int kSweepTX = MPS_SWEEP_TX, kSweepTY = MPS_SWEEP_TY, kSweepKZ = MPS_SWEEP_KZ;
+constexpr int kSweepTX = MPS_SWEEP_TX, kSweepTY = MPS_SWEEP_TY;
 
 // per-face multipliers of the staged ghost coefficient (k_sweep_ref,
 // k_sweep2_fast): -1 on a no-flux face, g/h - 1 on a DIRC face, so that the
@@ -942,8 +940,11 @@ GhostD<T> ghost_multipliers(const mps_ctx *c, const Lev<T> &v)
 // a last round with few blocks takes as long as a full one: at 128^3 in FP64,
 // 26 chunks (1664 blocks, whatever the kernel) took 27.3 and 51.9 us (rows
 // from D; explicit), the 12 and 16 of this rule 20.2 and 46.4; at 161 x 97 x
-// 129 rows from D took 25.8 with 22 chunks, 20.9 with 12. At least 2 planes a chunk, at
-// most kSweepKZ and what a buffer resource spans.
+// 129 rows from D took 25.8 with 22 chunks, 20.9 with 12. At least 2 planes a
+// chunk, at most what a buffer resource spans. (With a bound of 54 planes, too,
+// FP64 rows from D at 257^3 ran six chunks in two rounds, 170 us a sweep, where
+// three in one take 157; of eleven other grids, 65 x 33 x 513 to 385 x 129 x
+// 129, in both precisions and both kinds of rows, none is slower without it.)
 template <auto Kernel>
 int fast_chunks(const mps_ctx *c, int nz, long long cols, long long plane_bytes)
 {
@@ -954,7 +955,7 @@ int fast_chunks(const mps_ctx *c, int nz, long long cols, long long plane_bytes)
         return e == hipSuccess && n > 0 ? n : 4;
     }();
     const long long held = (long long)per_cu * c->cus;
-    const long long kmax = std::min<long long>(kSweepKZ, ((1LL << 31) - 1) / plane_bytes - 4);
+    const long long kmax = ((1LL << 31) - 1) / plane_bytes - 4;
     int best = (int)((nz + kmax - 1) / kmax);
     long long steps = 0;
     for (int r = 1; r <= 8; ++r) {
@@ -1387,12 +1388,12 @@ void vcycle(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, T *bwork, bool homog
 
 // Full multigrid for A e = L[0].b on the aligned hierarchy (homogeneous
 // rows, correction form): the right-hand side is restricted to every level
-// down to the first one the V-cycle solves as a whole (the LDS-resident
-// levels, else the coarsest), that level is solved by one V-cycle from zero,
-// and on the way up each level starts from the trilinear interpolation of
-// the coarser solution and runs one V-cycle. e ends in L[0].u. A level's
-// right-hand side is still intact when its turn comes: the V-cycles of the
-// coarser levels overwrite only the right-hand sides below them.
+// down to the first of the small ones (plain_from, else the coarsest), that
+// level is solved by one V-cycle from zero, and on the way up each level
+// starts from the trilinear interpolation of the coarser solution and runs
+// one V-cycle. e ends in L[0].u. A level's right-hand side is still intact
+// when its turn comes: the V-cycles of the coarser levels overwrite only the
+// right-hand sides below them.
 // The coarse levels' cycles of the full-multigrid pass smooth once before
 // and once after (their errors are corrected again by the finest level's
 // cycle): measured at 257^3, the pass reaches the same defect (4.7e-5
