@@ -1293,26 +1293,21 @@ void launch_tail(mps_ctx *c, std::vector<LevelBuf<T>> &L, int l, bool homog, boo
         A.rows[q] = L[l + q].rows;
         for (int f = 0; f < 6; ++f) A.face[q][f] = homog ? nullptr : L[l + q].faces[f];
     }
-    auto go = [&](auto O, auto V, auto R, auto F) {
+    // (the rows are formed: reaction and time terms are in their diagonals)
+    auto go = [&](auto O, auto V, auto F) {
+        constexpr int op = decltype(O)::value;
+        constexpr bool vel = decltype(V)::value, lin = decltype(F)::value;
         if (up)
-            hipLaunchKernelGGL((k_tail_up<T, decltype(O)::value, decltype(V)::value, decltype(R)::value,
-                                          decltype(F)::value>),
-                               dim3(1), dim3(kTailThreads), 0, c->stream, A);
+            hipLaunchKernelGGL((k_tail_up<T, op, vel, lin>), dim3(1), dim3(kTailThreads), 0, c->stream, A);
         else
-            hipLaunchKernelGGL((k_tail_down<T, decltype(O)::value, decltype(V)::value, decltype(R)::value,
-                                            decltype(F)::value>),
-                               dim3(1), dim3(kTailThreads), 0, c->stream, A);
+            hipLaunchKernelGGL((k_tail_down<T, op, vel, lin>), dim3(1), dim3(kTailThreads), 0, c->stream, A);
     };
-    const bool fast = A.L[0].fast != 0;   // rows without convection only
     const BoolC<true> yes{};
     const BoolC<false> no{};
-    if (level_op(c, L, l) == OP_STENCIL) go(IntC<OP_STENCIL>{}, no, no, yes);
-    else if (fast && c->has_reac) go(IntC<OP_REF>{}, no, yes, yes);
-    else if (fast) go(IntC<OP_REF>{}, no, no, yes);
-    else if (c->has_vel && c->has_reac) go(IntC<OP_REF>{}, yes, yes, no);
-    else if (c->has_vel) go(IntC<OP_REF>{}, yes, no, no);
-    else if (c->has_reac) go(IntC<OP_REF>{}, no, yes, no);
-    else go(IntC<OP_REF>{}, no, no, no);
+    if (level_op(c, L, l) == OP_STENCIL) go(IntC<OP_STENCIL>{}, no, yes);
+    else if (A.L[0].fast) go(IntC<OP_REF>{}, no, yes);   // rows without convection only
+    else if (c->has_vel) go(IntC<OP_REF>{}, yes, no);
+    else go(IntC<OP_REF>{}, no, no);
 }
 
 // --------------------------------------------------------------- V-cycle

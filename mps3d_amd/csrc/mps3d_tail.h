@@ -75,7 +75,7 @@ struct TailCell : TailPlace {
     T k[NK], v[NV];
 };
 
-template <typename T, int OP, bool VEL, bool REAC, bool LIN>
+template <typename T, int OP, bool VEL, bool LIN>
 struct Tail {
     static constexpr bool GL = !LIN;   // exact rows: face conductances in LDS
     static constexpr int NK = GL ? 1 : 6, NV = VEL ? 6 : 1;
@@ -248,10 +248,10 @@ __global__ void __launch_bounds__(kBlock) k_tail_rows(TailLevels<T> A)
     }
 }
 
-template <typename T, int OP, bool VEL, bool REAC, bool LIN>
+template <typename T, int OP, bool VEL, bool LIN>
 __global__ void __launch_bounds__(kTailThreads) k_tail_down(TailLevels<T> A)
 {
-    using K = Tail<T, OP, VEL, REAC, LIN>;
+    using K = Tail<T, OP, VEL, LIN>;
     using Cell = typename K::Cell;
     __shared__ typename K::Lds S;
     const int tid = threadIdx.x;
@@ -353,10 +353,10 @@ __global__ void __launch_bounds__(kTailThreads) k_tail_down(TailLevels<T> A)
     }
 }
 
-template <typename T, int OP, bool VEL, bool REAC, bool LIN>
+template <typename T, int OP, bool VEL, bool LIN>
 __global__ void __launch_bounds__(kTailThreads) k_tail_up(TailLevels<T> A)
 {
-    using K = Tail<T, OP, VEL, REAC, LIN>;
+    using K = Tail<T, OP, VEL, LIN>;
     using Cell = typename K::Cell;
     __shared__ typename K::Lds S;
     const int tid = threadIdx.x;
