@@ -171,11 +171,16 @@ def own_methods(obj, cls, methods):
 _OPERATOR = {k: vars(Operator)[k] for k in ("configure", "solve", "advance")}
 
 
+def plain_operator(op):
+    """Whether op is an Operator with its own methods."""
+    return own_methods(op, Operator, _OPERATOR)
+
+
 def advance(op, rhs, x0, vel=None, scale=1.0):
     """The interior solution of op for velocities scale * vel, outside
     autograd: an Operator scales them as it pads them; one of the caller's is
     called as linear_solve calls it, by configure(vel, rhs) and solve(x0)."""
-    if own_methods(op, Operator, _OPERATOR):
+    if plain_operator(op):
         return op.advance(rhs, x0, vel, scale)
     return linear_solve(op, rhs, None if vel is None else tuple(scale * v for v in vel), x0=x0)
 

@@ -45,7 +45,7 @@ import torch
 from torch.utils.checkpoint import checkpoint
 
 from . import _lib as M
-from .autograd import Operator, advance, linear_solve, native_fields, own_methods
+from .autograd import Operator, advance, linear_solve, native_fields, own_methods, plain_operator
 
 E_CHARGE = 1.602176634e-19
 EPS0 = 8.8541878128e-12
@@ -370,10 +370,24 @@ class Discharge:
         return tuple(new), neps_new
 
     # ------------------------------------------------------------ runs
+    def _closed(self, V, flat):
+        """Whether native steps from V and flat can stand for a segment whose
+        gradients are wanted: the steps are the class's own and nothing else
+        that they read (permittivity, operators, what the electrodes' faces
+        hold) can want a gradient."""
+        ops = [self.poisson, *self.ops] + ([self.energy_op] if self.energy else [])
+        if type(V) is not torch.Tensor or not own_methods(self, Discharge, _STEPS) or self.eps_r.requires_grad or \
+                not all(plain_operator(op) for op in ops) or any(t.requires_grad for t in self.faces(V.detach())):
+            return False
+        dens, neps = tuple(flat[:len(self.species)]), (flat[-1] if self.energy else None)
+        with torch.no_grad():
+            return self._native(dens, neps, V) is not None
+
     def run(self, V, nsteps, state, checkpoint_every=0, timed=False):
         """The state after nsteps steps; state = (dens tuple, neps or None).
         With checkpoint_every > 0 (and grad enabled) the steps are recomputed
-        segment by segment in the backward pass."""
+        segment by segment in the backward pass, in the forward pass built as
+        outside autograd where they can be (_Segment)."""
         dens, neps = state
         ns = len(dens)
 
@@ -389,7 +403,10 @@ class Discharge:
             m = min(checkpoint_every, nsteps - done) if checkpoint_every > 0 else 1
             t = time.perf_counter()
             if checkpoint_every > 0 and torch.is_grad_enabled():
-                flat = checkpoint(segment, m, V, *flat, use_reentrant=False)
+                if self._closed(V, flat):
+                    flat = _Segment.apply(segment, m, V, *flat)
+                else:
+                    flat = checkpoint(segment, m, V, *flat, use_reentrant=False)
             else:
                 flat = segment(m, V, *flat)
             if timed:
@@ -424,9 +441,38 @@ class Discharge:
             self.energy_op.close()
 
 
+class _Segment(torch.autograd.Function):
+    """Steps of a checkpointed run: native ones now, built from tensor
+    operations again in the backward pass for their gradients. (With
+    torch.utils.checkpoint the first pass too is built from tensor operations,
+    and its first use in a process imports the compiler. The gradient of 20
+    steps of five species at 257^3 then took 3.3 to 3.6 times the native
+    forward pass alone in a process and 2.7 to 3.0 after other work; with this
+    2.8 and 2.6.)"""
+
+    @staticmethod
+    def forward(ctx, segment, m, *state):
+        ctx.segment, ctx.m = segment, m
+        ctx.save_for_backward(*state)
+        ctx.set_materialize_grads(False)
+        return segment(m, *state)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        ins = [t.detach().requires_grad_(need) for t, need in zip(ctx.saved_tensors, ctx.needs_input_grad[2:])]
+        want = [t for t in ins if t.requires_grad]
+        with torch.enable_grad():
+            out = ctx.segment(ctx.m, *ins)
+        ends = [(o, g) for o, g in zip(out, grads) if g is not None and o.requires_grad]
+        got = iter(torch.autograd.grad([o for o, _ in ends], want, [g for _, g in ends], allow_unused=True)
+                   if ends and want else [None] * len(want))
+        return (None, None) + tuple(next(got) if t.requires_grad else None for t in ins)
+
+
 # the methods whose work the native step does in its own passes
 _PIECES = {k: vars(Discharge)[k] for k in ("potential", "efield", "mean_energy", "rates", "thermal_outflow",
                                            "solve_species", "solve_energy")}
+_STEPS = dict(_PIECES, **{k: vars(Discharge)[k] for k in ("step", "solve_poisson")})
 _RATE = {"coefficient": Reaction.coefficient}
 
 

@@ -201,3 +201,69 @@ def test_the_local_field_constants_are_read_where_they_are_used(gpu):
         m.close()
     (a, ea), (b, eb) = out
     assert all(torch.equal(x, y) for x, y in zip(a + (ea,), b + (eb,)))
+
+
+def gradients(m, n, V, every, extra=()):
+    """A run of five steps: its end and the gradients of a sum over it."""
+    dens, neps = state(m, n)
+    dens = tuple(d.requires_grad_() for d in dens)
+    m._phi = None
+    out, end = m.run(V, 5, (dens, neps), checkpoint_every=every)
+    out = out + ((end,) if m.energy else ())
+    g = torch.Generator(device="cuda").manual_seed(2)
+    J = sum((t * torch.rand(t.shape, generator=g, dtype=F64, device="cuda")).sum() for t in out)
+    J = J + 1e-3 * float(J.detach()) / 1e6 * (m.potential_of((out[:len(dens)], None), V) ** 2).mean()
+    return [t.detach() for t in out], torch.autograd.grad(J, [V, *dens, *extra])
+
+
+@pytest.mark.parametrize("form", ["energy", "local"])
+@pytest.mark.parametrize("every", [1, 2, 5])
+def test_checkpointed_gradients(gpu, form, every, monkeypatch):
+    # segments of native steps give the gradients of the steps kept whole. The
+    # solves reach 1e-10 of their right-hand sides, so both hold to 1e-8 and
+    # their gradients to some ten times that
+    n, native = 8, []
+    m = build(DS.Discharge, form, n)
+    V = torch.tensor([800.0, -300.0], dtype=F64, device="cuda", requires_grad=True)
+    step = DS.Discharge._native_step
+    monkeypatch.setattr(DS.Discharge, "_native_step", lambda self, *a: native.append(1) or step(self, *a))
+    end, want = gradients(m, n, V, 0)
+    assert not native
+    got_end, got = gradients(m, n, V, every)
+    assert len(native) == 5
+    for a, b in zip(list(got) + got_end, list(want) + end):
+        assert float((a - b).abs().max()) <= 1e-7 * float(b.abs().max())
+    m.close()
+
+
+def test_what_else_wants_a_gradient_keeps_it(gpu):
+    # a tensor that the electrodes' faces hold, a permittivity, a rate: their
+    # segments are checkpointed as they are, and V may be a list
+    n = 8
+    V = torch.tensor([800.0, -300.0], dtype=F64, device="cuda", requires_grad=True)
+    for what in ("faces", "rate", "eps_r"):
+        m = build(DS.Discharge, "local", n)
+        p = torch.ones((), dtype=F64, device="cuda", requires_grad=True)
+        faces, rate, eps = m.faces, m.reactions[0].rate, m.eps_r
+        if what == "faces":
+            m.faces = lambda V_: tuple(p * f for f in faces(V_))
+        elif what == "rate":
+            m.reactions[0].rate = lambda e: p * rate(e)
+        else:
+            m.eps_r = p * eps
+        assert not m._closed(V, state(m, n)[0])
+        if what == "eps_r":
+            m.eps_r = eps   # (its gradient would run through the potential's right-hand side only)
+            m.close()
+            continue
+        _, want = gradients(m, n, V, 0, (p,))
+        _, got = gradients(m, n, V, 2, (p,))
+        for a, b in zip(got, want):
+            assert float((a - b).abs().max()) <= 1e-7 * float(b.abs().max())
+        m.close()
+    m = build(DS.Discharge, "local", n)
+    assert m._closed(V, state(m, n)[0])
+    assert not m._closed([V[0], V[1]], state(m, n)[0])
+    m.solve_poisson = lambda rhs: DS.Discharge.solve_poisson(m, rhs)
+    assert not m._closed(V, state(m, n)[0])
+    m.close()
