@@ -941,10 +941,12 @@ GhostD<T> ghost_multipliers(const mps_ctx *c, const Lev<T> &v)
 // 26 chunks (1664 blocks, whatever the kernel) took 27.3 and 51.9 us (rows
 // from D; explicit), the 12 and 16 of this rule 20.2 and 46.4; at 161 x 97 x
 // 129 rows from D took 25.8 with 22 chunks, 20.9 with 12. At least 2 planes a
-// chunk, at most what a buffer resource spans. (With a bound of 54 planes, too,
-// FP64 rows from D at 257^3 ran six chunks in two rounds, 170 us a sweep, where
-// three in one take 157; of eleven other grids, 65 x 33 x 513 to 385 x 129 x
-// 129, in both precisions and both kinds of rows, none is slower without it.)
+// chunk, at most what a buffer resource spans. Within a solve at 257^3: FP64
+// rows from D 187 us a sweep with 15 chunks, 175 with six in two rounds, 160
+// with the three in one round of this rule; FP32 94.5 with 15 and with its
+// five. (Of eleven other grids, 65 x 33 x 513 to 385 x 129 x 129, in both
+// precisions and both kinds of rows, none is slower than with at most 54
+// planes a chunk.)
 template <auto Kernel>
 int fast_chunks(const mps_ctx *c, int nz, long long cols, long long plane_bytes)
 {

@@ -875,7 +875,7 @@ __global__ void __launch_bounds__(kBlock) k_sg_stencil(Lev<double> L, RowArrays 
 // operator is singular depends on how its elimination rounds, and the caller
 // leaves the answer, and the inverse, to host_bottom_inverse.
 // 27 cells 21 us, 64 cells 52 us (98 us with the matrix in LDS, one column
-// per lane), 128 cells 162 us, 210 cells 453 us (2.2 us per pivot; 1024 lanes
+// per lane), 128 cells 162 us, 210 cells 444 us (2.1 us per pivot; 1024 lanes
 // with 49 entries each spill: 1000 us). On the host, with the rows copied
 // there and the inverse back, the 210-cell one held a 6.6 ms species step up
 // for more than 2 ms.

@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(THREADS) k_small_cycle(SmallLevels<T> A)
         for (int p = 0; p < 2; ++p)
             if (cells[p].q >= 0) V.b[cells[p].q] = bo[p];
     }
-    // coarsest level: u = A^-1 b (at most half the workgroup's rows)
+    // coarsest level: u = A^-1 b (no more rows than lanes)
     {
         const SmallView<T> V = small_view(A, mem, last);
         double s = 0.0;
