@@ -21,6 +21,7 @@ import ctypes as C
 
 import torch
 from torch.autograd import forward_ad as fwAD
+from torch.utils._device import DeviceContext
 
 from . import _lib as M
 from .solver import FieldSolver
@@ -38,11 +39,15 @@ def interior(g):
 def native_fields(shape, *fields):
     """Whether the library's field passes can take these tensors by address:
     contiguous float64 fields of that shape on the current GPU, outside
-    tracing, functorch transforms, forward-mode levels and dispatch modes
-    (which see tensor operations only)."""
+    tracing, functorch transforms, forward-mode levels, dispatch modes and
+    function modes other than a default device (which see tensor operations
+    only)."""
     if torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active():
         return False
     if fwAD._current_level >= 0 or torch._C._len_torch_dispatch_stack() or max(shape) > 16000:
+        return False
+    if any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+           for i in range(torch._C._len_torch_function_stack())):
         return False
     dev = torch.cuda.current_device()
     return all(type(t) is torch.Tensor and t.is_cuda and t.device.index == dev and t.dtype == torch.float64 and

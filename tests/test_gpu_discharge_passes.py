@@ -267,3 +267,28 @@ def test_what_else_wants_a_gradient_keeps_it(gpu):
     m.solve_poisson = lambda rhs: DS.Discharge.solve_poisson(m, rhs)
     assert not m._closed(V, state(m, n)[0])
     m.close()
+
+
+def test_function_modes_see_the_tensor_operations(gpu):
+    # as dispatch modes do; a default device is no such mode
+    from torch.overrides import TorchFunctionMode
+
+    class Hot(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            return 2.0 * out if func is torch.exp else out
+
+    out, V = [], torch.tensor([800.0], dtype=F64, device="cuda")
+    for cls in (DS.Discharge, Torch):
+        m = build(cls, "energy", 8)
+        dens, neps = state(m, 8)
+        with torch.device("cuda"):
+            assert (m._native(dens, neps, V) is not None) == (cls is DS.Discharge)
+        with Hot():
+            native = m._native(dens, neps, V)
+            new, end = m.step(dens, neps, V)
+        out.append(new + (end,))
+        m.close()
+        assert native is None
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
